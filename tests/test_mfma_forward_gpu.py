@@ -1,0 +1,130 @@
+"""GPU parity of the matrix-core one-launch forward (the bf16 inference forward where one round of
+workgroups holds every segment) at the sizes where its blocks, chunks and head groups end, against the
+fp64 oracle on the same rounded inputs.
+
+Tolerances: y is rounded once to bf16, 2^-9 of the value, so 2^-8 of the largest value leaves as much
+again for the sums; the state is fp32 throughout with operands split to 2^-24, the dynamics' hardware
+log / exp (2e-5) being the largest error, so 5e-5 of the largest state value.
+"""
+
+import pytest
+import torch
+
+from _gpu_util import DEV, ScanConfig, draw_inputs, log, oracle_fwd, rel, to_dev
+from oracle import cdssm_oracle as o
+
+pytestmark = pytest.mark.gpu
+
+TOL_Y, TOL_H = 2.0 ** -8, 5e-5
+KEYS = ("q", "k", "v", "beta", "sel_C", "dt", "r", "alpha", "omega")
+
+
+def run(x, chunk=None):
+    from cdssm_hip import check_lookback, chunkwise_delta_scan
+    y, h = chunkwise_delta_scan(*[x[n] for n in KEYS], x["c"], h0=x.get("h0"), chunk_size=chunk)
+    torch.cuda.synchronize()
+    check_lookback()
+    return y.cpu(), h.cpu()
+
+
+@pytest.mark.parametrize("B,H,L,D,chunk", [
+    (1, 1, 1, 64, None), (2, 3, 15, 64, None), (1, 4, 16, 64, None), (1, 5, 17, 64, None), (1, 8, 64, 64, None),
+    (3, 6, 65, 64, None), (1, 4, 257, 64, None), (2, 7, 100, 64, 1), (1, 4, 130, 64, 17), (1, 6, 300, 64, 128),
+    (1, 2, 1, 128, None), (2, 5, 127, 128, None), (1, 4, 513, 128, None), (1, 3, 200, 128, 48)])
+def test_matches_oracle_at_the_edges_of_blocks_chunks_and_head_groups(B, H, L, D, chunk):
+    log(f"[mfma forward] B{B} H{H} L{L} D{D} chunk={chunk or D}")
+    x = draw_inputs(ScanConfig("t", B=B, H=H, L=L, D=D, h0_std=0.1), seed=L + H)
+    y, h = run(to_dev(x), chunk)
+    yr, hr = oracle_fwd(x, chunk)
+    assert rel(y, yr) <= TOL_Y and rel(h, hr) <= TOL_H, (rel(y, yr), rel(h, hr))
+
+
+@pytest.mark.parametrize("alpha,omega", [(3.0, 0.02), (1.0, 0.0), (10.0, 0.1)])
+@pytest.mark.parametrize("D", [64, 128])
+def test_strong_decay_runs_blocks_in_true_units(D, alpha, omega):
+    """|a_t| far below 2^-5: the products of a over 16 tokens underflow their reciprocal, so most blocks run
+    the true-units solve."""
+    log(f"[mfma forward] strong decay D{D} alpha x{alpha} omega x{omega}")
+    x = draw_inputs(ScanConfig("t", B=1, H=6, L=300, D=D, h0_std=0.1), seed=3)
+    x["alpha"], x["omega"] = x["alpha"] * alpha, x["omega"] * omega
+    y, h = run(to_dev(x))
+    yr, hr = oracle_fwd(x)
+    assert rel(y, yr) <= TOL_Y and rel(h, hr) <= TOL_H, (rel(y, yr), rel(h, hr))
+
+
+@pytest.mark.parametrize("N", [2, 4, 6, 16])
+def test_gate_level_rows_match_oracle(N):
+    """State rows as virtual heads: 4 consecutive ones of a wave may share a key head or not (N / 2 = 1, 2, 3, 8)."""
+    from cdssm_hip import chunkwise_delta_scan_abar
+    B, H, L, D = 2, 3, 150, 64
+    log(f"[mfma forward] gate level N={N}")
+    g = torch.Generator().manual_seed(N)
+    n = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    q, k = (torch.nn.functional.normalize(n(B, L, H, D), dim=-1) for _ in range(2))
+    A = torch.polar(torch.sigmoid(n(B, L, H, N // 2) + 2), n(B, L, H, N // 2))
+    x = [t.bfloat16() for t in (q, k, n(B, L, H, N), torch.sigmoid(n(B, L, H)), torch.sigmoid(n(B, L, H)),
+                                torch.view_as_real(A).flatten(-2), torch.sigmoid(n(B, L, H, N // 2)))]
+    h0 = 0.1 * n(B, H, N, D)
+    y, h = chunkwise_delta_scan_abar(*[t.to(DEV) for t in x], h0=h0.to(DEV))
+    q, k, v, beta, sel, A, vp = [t.double() for t in x]
+    Y, hr = o.ssd_chunkwise_scan(A, k, v * vp.repeat_interleave(2, dim=-1), beta, D, N, h0=h0.double(),
+                                 return_final=True)
+    yr = o.readout(Y, q, sel)
+    assert rel(y, yr) <= TOL_Y and rel(h, hr) <= 1e-6 * 4, (rel(y, yr), rel(h, hr))
+
+
+def test_misaligned_scalars_take_the_element_loads():
+    """beta, sel_C, dt, r and v one element off their 8-byte (4-byte) alignment: the same values, bit for bit."""
+    x = to_dev(draw_inputs(ScanConfig("t", B=2, H=8, L=333, D=64), seed=1))
+    ref = run(x)
+    for n in ("v", "beta", "sel_C", "dt", "r"):
+        t = torch.empty(x[n].numel() + 1, dtype=x[n].dtype, device=DEV)[1:].view(x[n].shape)
+        x[n] = t.copy_(x[n])
+        assert x[n].data_ptr() % 4 == 2
+    got = run(x)
+    assert torch.equal(ref[0], got[0]) and torch.equal(ref[1], got[1])
+
+
+@pytest.mark.parametrize("name,value", [("k", float("nan")), ("k", float("inf")), ("q", float("nan")),
+                                        ("v", float("inf")), ("dt", float("nan"))])
+def test_non_finite_input_stays_in_its_head(name, value):
+    """One non-finite element in head 1 at token 37: the other heads of the wave are bit-identical to a clean
+    run's, head 1 is so before that token and non-finite at it (q: at it only)."""
+    B, H, L, t, h = 1, 4, 150, 37, 1
+    log(f"[mfma forward] {value} in {name}")
+    x = to_dev(draw_inputs(ScanConfig("t", B=B, H=H, L=L, D=64), seed=2))
+    y0, h0 = run(x)
+    x[name] = x[name].clone()
+    x[name][0, t, h].view(-1)[0] = value
+    y1, h1 = run(x)
+    rest = [i for i in range(H) if i != h]
+    assert torch.equal(y0[:, :, rest], y1[:, :, rest]) and torch.equal(h0[:, rest], h1[:, rest])
+    assert torch.equal(y0[:, :t, h], y1[:, :t, h])
+    assert not y1[:, t, h].isfinite().any()
+    if name == "q":
+        assert torch.equal(y0[:, t + 1:, h], y1[:, t + 1:, h]) and torch.equal(h0, h1)
+    else:
+        assert not y1[:, -1, h].isfinite().any() and not h1[:, h].isfinite().any()
+
+
+def test_continuing_call_after_a_four_launch_training_call():
+    """A *_continue inference call on a workspace whose previous call was a training forward of the shape, which
+    takes four launches here (more segments of 8 heads than compute units): the look-back epoch is there."""
+    from cdssm_hip import _lib, check_lookback
+    from cdssm_hip.scan import PreparedForward
+    x = to_dev(draw_inputs(ScanConfig("t", B=1, H=20, L=64 * 4 * 90, D=64), seed=4))
+    args = [x[n] for n in KEYS]
+    train, infer = PreparedForward(*args, x["c"], train=True), PreparedForward(*args, x["c"])
+    infer()
+    torch.cuda.synchronize()
+    y, h = infer.y.clone(), infer.h_final.clone()
+    train()
+    a = list(infer._args)
+    a[-7] = _lib.ptr(train.workspace)
+    for _ in range(3):
+        infer.y.zero_()
+        st = infer._lib.cdssm_fused_scan_fwd_continue(*a, _lib.stream_of(DEV))
+        assert st == 0
+        torch.cuda.synchronize()
+        check_lookback()
+        assert torch.equal(infer.y, y) and torch.equal(infer.h_final, h)
