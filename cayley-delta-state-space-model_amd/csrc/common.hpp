@@ -573,12 +573,12 @@ constexpr uint64_t kSpinTicks = 5000000;  // look-back wait bound: 50 ms of the 
 // complex + one complex scalar), a state (D complex) and an 8-byte flag, then
 // a control block of kCtlWords 8-byte words whose first word is the call's
 // epoch and second a count of workgroups.  The area is never cleared: a flag
-// counts only when its upper bits equal the epoch of the running call, which
-// a one-thread kernel launched just before the pass draws from a device-side
-// counter and writes into the control block, or, for the *_continue calls,
-// the previous call left there (arrive_and_draw_next_epoch).  Drawing it on
-// the device keeps a captured HIP graph correct: every replay gets a new
-// epoch.
+// counts only when its upper bits equal the epoch of the running call: drawn on
+// the host and passed as an argument where the call is launched eagerly (a
+// launch less: 2-5 us on the GPU); in a captured call drawn by a one-thread
+// kernel launched just before the pass from a device-side counter, so that
+// every replay gets a new one; for the *_continue calls the one the previous
+// call left in the control block (leave_next_epoch).
 struct OnePassBufs {
   float2* seg_f;             // (B, NSEG, H, D) segment map F: state at the segment's end from zero
   float2* seg_s;             // (B, NSEG, H, D) state leaving the segment
@@ -588,6 +588,7 @@ struct OnePassBufs {
   // forward only (two-level fold): (B, NGRP, H, D) group map F and (B, NGRP, H) its rotation product
   float2* grp_f = nullptr;
   float2* grp_g = nullptr;
+  unsigned long long epoch = 0;  // the call's epoch drawn on the host, or 0: ctl[0] holds it
 };
 
 // Epoch words: the pass's tag in bits 58..59 (so epochs of different passes
@@ -619,6 +620,21 @@ __device__ __forceinline__ void arrive_and_draw_next_epoch(unsigned long long* c
     const unsigned long long n = __hip_atomic_fetch_add(calls, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1ull;
     __hip_atomic_store(ctl + 1, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __hip_atomic_store(ctl, epoch_word(tag, n), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+// The running call's epoch: drawn on the host for a call launched eagerly (no launch of its own), else the
+// control block's (captured calls, whose replays each need a new one, and the *_continue calls).
+__device__ __forceinline__ unsigned long long call_epoch(const OnePassBufs& ob) {
+  return ob.epoch ? ob.epoch : load_epoch(ob.ctl);
+}
+// Once per workgroup, after its first flag: leave the next call's epoch in the control block.
+__device__ __forceinline__ void leave_next_epoch(const OnePassBufs& ob, unsigned long long* calls, unsigned tag) {
+  if (!ob.epoch) {
+    arrive_and_draw_next_epoch(ob.ctl, calls, tag);
+  } else if (blockIdx.x == 0) {  // no workgroup of this call reads the control block
+    const unsigned long long n = __hip_atomic_fetch_add(calls, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1ull;
+    __hip_atomic_store(ob.ctl + 1, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(ob.ctl, epoch_word(tag, n), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 // Bits of the sticky look-back status word (cdssm_lookback_status).
@@ -656,6 +672,10 @@ int bwd_lookback_status(bool clear, unsigned* out);
 // Workgroups of kernel `fn` (block threads, lds bytes of dynamic LDS) resident
 // on the current device at once; 0 if it cannot run.  Cached.
 int resident_capacity(const void* fn, int block, size_t lds);
+// A look-back epoch for a call about to be launched eagerly on `stream`: unique in the process, apart from
+// the device-drawn ones (bit 57 of the count).  0 while the stream is being captured (a replay would repeat
+// it) or cannot be asked: the call then draws its epoch on the device.
+unsigned long long draw_call_epoch(unsigned tag, hipStream_t stream);
 // Compute units of the current device (0 if it cannot be read).  Cached.
 int device_cus();
 // Launch-path selection of the fused scan (forward and backward carry):

@@ -647,7 +647,7 @@ __global__ __launch_bounds__(kWave * kOnePassW) void fused_bwd_corrcarry_kernel(
   static_assert(EPT >= 1 && EPT * kWave * W == SEGN && D % EPT == 0, "segment state tiles the workgroup");
   extern __shared__ float4 smem4[];
   const int L = a.L, H = a.H, Q = a.Q, NC = a.NC, NSEG = a.NSEG;
-  const unsigned long long epoch = load_epoch(a.ob.ctl);
+  const unsigned long long epoch = call_epoch(a.ob);
 
   const int wv = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / kWave);
   const int lane = int(threadIdx.x) % kWave;
@@ -818,7 +818,7 @@ __global__ __launch_bounds__(kWave * kOnePassW) void fused_bwd_corrcarry_kernel(
   if (threadIdx.x == 0) {
     __hip_atomic_store(flag, (epoch << 2) | 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     // every workgroup of the grid holds this call's epoch once all have published
-    arrive_and_draw_next_epoch(ob.ctl, &g_bwd_calls, 2u);
+    leave_next_epoch(ob, &g_bwd_calls, 2u);
   }
 
   stamp(3);
@@ -1909,7 +1909,8 @@ int launch_fused_bwd(const void* q, const void* k, const void* v, const void* be
         a.stamps = t_bstamps.buf;
       }
       // a continuing call runs on the epoch the previous call's last workgroup left
-      if (!cont) {
+      if (!cont) a.ob.epoch = cdssm_host::draw_call_epoch(2u, stream);
+      if (!cont && !a.ob.epoch) {
         hipLaunchKernelGGL(bwd_epoch_kernel, dim3(1), dim3(64), 0, stream, a.ob.ctl);
         st = cdssm_host::check_launch("cdssm_fused_scan_bwd/epoch");
         if (st) return st;

@@ -1356,7 +1356,7 @@ __device__ __forceinline__ void onepass_segment(const OnePassArgs<T>& a, int ite
 template <typename T, int D, int LPH, bool SAVE, bool PERSIST, bool WIDE = false>
 __global__ __launch_bounds__(kWave * kOnePassW) void fused_fwd_onepass_kernel(OnePassArgs<T> a) {
   // read once: the call's last workgroup to have read it stores the next call's
-  const unsigned long long epoch = load_epoch(a.ob.ctl);
+  const unsigned long long epoch = call_epoch(a.ob);
   if (!PERSIST) {
     onepass_segment<T, D, LPH, SAVE, WIDE>(a, int(blockIdx.x), epoch, true);
     return;
@@ -1569,7 +1569,8 @@ int launch_fused_fwd(const void* q, const void* k, const void* v, const void* be
       }
       if (path) *path = cdssm_host::kPathOne;
       // a continuing call runs on the epoch the previous call's last workgroup left
-      if (!cont) {
+      if (!cont) a.ob.epoch = cdssm_host::draw_call_epoch(1u, stream);
+      if (!cont && !a.ob.epoch) {
         hipLaunchKernelGGL(fwd_epoch_kernel, dim3(1), dim3(64), 0, stream, a.ob.ctl);
         const int est = cdssm_host::check_launch("cdssm_fused_scan_fwd/epoch");
         if (est) return est;

@@ -100,7 +100,7 @@ __device__ __forceinline__ void segment_carry(const OnePassBufs& ob, const float
     __syncthreads();
     if (threadIdx.x == 0) {
       __hip_atomic_store(flag, (epoch << 3) | bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (arrive) arrive_and_draw_next_epoch(ob.ctl, calls, tag);
+      if (arrive) leave_next_epoch(ob, calls, tag);
     }
   }
 
@@ -157,7 +157,7 @@ __device__ __forceinline__ void segment_carry(const OnePassBufs& ob, const float
     bits |= kFlagGroup;
     if (threadIdx.x == 0) {
       __hip_atomic_store(flag, (epoch << 3) | bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (arrive) arrive_and_draw_next_epoch(ob.ctl, calls, tag);
+      if (arrive) leave_next_epoch(ob, calls, tag);
     }
   }
 

@@ -810,7 +810,7 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
 // slower than that kernel from two rounds on (B1 H32 L65536 D64: 196-206 against 177 us).
 template <int D, bool ABAR>
 __global__ __launch_bounds__(kWave* kOnePassW, D == 64 ? 2 : 1) void mf_onepass_kernel(MfArgs a) {
-  mf_segment<D, ABAR>(a, int(blockIdx.x), load_epoch(a.ob.ctl));
+  mf_segment<D, ABAR>(a, int(blockIdx.x), call_epoch(a.ob));
 }
 
 template <int D, bool ABAR>
@@ -863,7 +863,8 @@ int mf_launch(const MfmaForward& p, hipStream_t stream, hipEvent_t* ev) {
     }
     a.stamps = p.stamps;
   }
-  if (!p.cont) {
+  if (!p.cont) a.ob.epoch = cdssm_host::draw_call_epoch(kMfTag, stream);
+  if (!p.cont && !a.ob.epoch) {
     hipLaunchKernelGGL(mf_epoch_kernel, dim3(1), dim3(64), 0, stream, a.ob.ctl);
     const int st = cdssm_host::check_launch("cdssm_fused_scan_fwd/epoch");
     if (st) return st;

@@ -59,6 +59,18 @@ int resident_capacity(const void* fn, int block, size_t lds) {
   return capacity;
 }
 
+unsigned long long draw_call_epoch(unsigned tag, hipStream_t stream) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &cap) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  if (cap != hipStreamCaptureStatusNone) return 0;
+  static std::atomic<unsigned long long> calls{0};
+  const unsigned long long n = calls.fetch_add(1, std::memory_order_relaxed) + 1;
+  return (static_cast<unsigned long long>(tag) << 58) | (1ull << 57) | (n & ((1ull << 57) - 1));
+}
+
 int device_cus() {
   int dev = 0, n_cu = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) {
