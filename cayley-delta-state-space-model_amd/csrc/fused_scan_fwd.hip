@@ -1853,16 +1853,18 @@ int fused_fwd_entry(int dtype, const void* q, const void* k, const void* v, cons
     reg = full_regions(workspace, lay);
   }
   const int b = int(B), l = int(L), hh = int(H), qc = int(chunk);
-  // bf16 inference in the readout form: the matrix-core one-launch forward, where one round of resident
+  // bf16 scan-level inference: the matrix-core one-launch forward, where one round of resident
   // workgroups (2 per CU at D = 64, 1 at D = 128) takes every segment.  Measured on MI355X against the
   // better of the other two forms: D 64 H4 L512 39.6 -> 23.0 us, B8 H16 L2048 35.2 -> 28.1, B8 H16 L4096
   // (the largest single round) 43.4 -> 41.7; D 128 B4 H16 L2048 72.1 -> 65.2, L8192 94.0 -> 76.1; with
-  // more rounds it is the slower one (B1 H32 L65536 D64: 177 against 196 us, looping over segments)
-  if (dtype == 1 && !ssd && !save && cdssm_host::scan_path() == cdssm_host::kPathAuto &&
-      mfma_forward_fits(B, L, H, int(D), qc, abar)) {
+  // more rounds it is the slower one (B1 H32 L65536 D64: 177 against 196 us, looping over segments).  The
+  // gate-level form keeps the sequential kernel: a model's prefill feeds decode states whose bits a
+  // generation continues from, and 24 bf16 layers turn another order of sums into 1e-2 of those states
+  if (dtype == 1 && !ssd && !abar && !save && cdssm_host::scan_path() == cdssm_host::kPathAuto &&
+      mfma_forward_fits(B, L, H, int(D), qc)) {
     if (path) *path = cdssm_host::kPathOne;
     return launch_mfma_forward(MfmaForward{q, k, v, beta, sel_c, dt, r, alpha, omega, c, h0, y, h_final, reg.onepass, b,
-                                           l, hh, int(D), qc, int(R), abar, cont, t_stamps.buf, t_stamps.len},
+                                           l, hh, int(D), qc, cont, t_stamps.buf, t_stamps.len},
                                stream, ev);
   }
 #define CDSSM_FWD_ARGS q, k, v, beta, sel_c, dt, r, alpha, omega, c, h0, y, h_final, reg, b, l, hh, qc, stream, \

@@ -1,7 +1,6 @@
-// The one-launch inference forward on the matrix cores: bf16 inputs, one
-// complex value per head (state_dim 2, or each state row of a larger one as a
-// virtual head), fp32 states, R-mode semantics and look-back carry of
-// fused_fwd_onepass_kernel.
+// The one-launch inference forward on the matrix cores: scan-level bf16
+// inputs, state_dim 2 (one complex value per head), fp32 states, R-mode
+// semantics and look-back carry of fused_fwd_onepass_kernel.
 //
 // The sequential form runs every token's dot products and updates over D on
 // the VALU, one dependent step per token.  Here a chunk goes in blocks of 16
@@ -91,7 +90,7 @@ struct MfArgs {
   uint16_t* y;
   float* h_final;
   OnePassBufs ob;
-  int L, H, R, Q, NC, NSEG, B, n_hg;
+  int L, H, Q, NC, NSEG, B, n_hg;
   bool wide;  // 8-byte loads of the per-token scalars
   unsigned long long* stamps;
 };
@@ -227,7 +226,7 @@ __device__ __forceinline__ void mf_solve(const float (&L)[16], float& xr, float&
 // One segment of 4 chunks of a head group; idx enumerates (unit = segment of a batch row, head group) so
 // that the head groups of a unit, which share the lines of the per-token scalars, lie 8 apart (one XCD
 // under the round-robin placement of workgroups) and lower segments come first.
-template <int D, bool ABAR>
+template <int D>
 __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned long long epoch) {
   using Cfg = MfCfg<D>;
   constexpr int KS = Cfg::KS, SROW = Cfg::SROW, W = kOnePassW, SEGN = kMfHeads * D;
@@ -246,7 +245,7 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
   const int hg = loc / width, unit = 8 * grp + (loc - hg * width);
   const int seg = unit / a.B, bi = unit - seg * a.B;
   const int hbase = hg * kMfHeads;
-  const int H = a.H, Hk = H / a.R, L = a.L, Q = a.Q;
+  const int H = a.H, L = a.L, Q = a.Q;
   const int n_live = min(W, a.NC - seg * W);
   const bool live = wv < n_live;
   const int chunk = min(seg * W + wv, a.NC - 1);
@@ -270,15 +269,15 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
   int* ctrl = reinterpret_cast<int*>(Sx + SEGN);
   if (threadIdx.x < Cfg::ZERO) zero[threadIdx.x] = 0u;
 
-  const int rowb = Hk * D * 2;  // bytes from token to token
+  const int rowb = H * D * 2;  // bytes from token to token
   int hoff[kMfHeads];
 #pragma unroll
-  for (int h = 0; h < kMfHeads; ++h) hoff[h] = (min(hbase + h, H - 1) / a.R) * D * 2;
-  const int64_t rest = int64_t(L - t0) * Hk * D * 2;
+  for (int h = 0; h < kMfHeads; ++h) hoff[h] = min(hbase + h, H - 1) * D * 2;
+  const int64_t rest = int64_t(L - t0) * H * D * 2;
   const uint32_t nrec = uint32_t(rest > 0xffffffffll ? 0xffffffffll : rest);
-  const auto krs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.k + row0 * Hk * D), short(0), int(nrec),
+  const auto krs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.k + row0 * H * D), short(0), int(nrec),
                                                      0x00020000);
-  const auto qrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.q + row0 * Hk * D), short(0), int(nrec),
+  const auto qrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.q + row0 * H * D), short(0), int(nrec),
                                                      0x00020000);
   auto voff = [&](int b) { return min(16 * b + i, tlast) * rowb + 16 * g; };
 
@@ -312,24 +311,22 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
   uint32_t exact = 0, marked = 0;  // bit b: block b runs in true units; holds a non-finite coefficient, beta or k
   float Gr = 1.0f, Gi = 0.0f;
   if (live) {
-    const float al = ABAR ? 0.0f : a.alpha[hl], om = ABAR ? 0.0f : a.omega[hl];
-    const int hk = hl / a.R;
+    const float al = a.alpha[hl], om = a.omega[hl];
 #pragma unroll 1
     for (int b0 = 0; b0 < nb; b0 += 4) {
-      float sb[4], ss[4], sd[4], sd2[4], sr4[4], sv0[4], sv1[4];
+      float sb[4], ss[4], sd[4], sr4[4], sv0[4], sv1[4];
       if (a.wide) {
-        // one 8-byte row (4 heads) of array g (beta, sel, dt or a_t, r or vp) per lane and token, and the
-        // token's v (and a_t) pair of the lane's own head; the 4 x 4 exchange between lane groups and heads
+        // one 8-byte row (4 heads) of array g (beta, sel, dt, r) per lane and token, and the
+        // token's v pair of the lane's own head; the 4 x 4 exchange between lane groups and heads
         // leaves each lane with its head's four scalars
         uint2 w4[4];
-        uint32_t pv[4], pa[4];
+        uint32_t pv[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           const int64_t tk = (row0 + min(16 * (b0 + u) + i, tlast)) * H;
-          const uint16_t* src = g == 0 ? a.beta : g == 1 ? a.sel : (g == 2 && !ABAR) ? a.dt : a.r;
+          const uint16_t* src = g == 0 ? a.beta : g == 1 ? a.sel : g == 2 ? a.dt : a.r;
           w4[u] = *reinterpret_cast<const uint2*>(src + tk + hbase);
           pv[u] = *reinterpret_cast<const uint32_t*>(a.v + 2 * (tk + hl));
-          pa[u] = ABAR ? *reinterpret_cast<const uint32_t*>(a.dt + 2 * (tk + hl)) : 0u;
         }
         if (b0 == 0) fk.load(krs, voff(0), hoff);
 #pragma unroll
@@ -341,22 +338,20 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
           swap16(x[2], x[3]);
           sb[u] = x[0];
           ss[u] = x[1];
-          sd[u] = ABAR ? bf16_lo(pa[u]) : x[2];
-          sd2[u] = ABAR ? bf16_hi(pa[u]) : 0.0f;
+          sd[u] = x[2];
           sr4[u] = x[3];
           sv0[u] = bf16_lo(pv[u]);
           sv1[u] = bf16_hi(pv[u]);
         }
       } else {
-      uint16_t rb[4], rs[4], rd[4], rd2[4], rr[4], rv0[4], rv1[4];
+      uint16_t rb[4], rs[4], rd[4], rr[4], rv0[4], rv1[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const int t = min(16 * (b0 + u) + i, tlast);
-        const int64_t e = (row0 + t) * H + hl, ek = (row0 + t) * Hk + hk;
-        rb[u] = a.beta[ek];
-        rs[u] = a.sel[ek];
-        rd[u] = ABAR ? a.dt[2 * e] : a.dt[e];
-        rd2[u] = ABAR ? a.dt[2 * e + 1] : uint16_t(0);
+        const int64_t e = (row0 + t) * H + hl;
+        rb[u] = a.beta[e];
+        rs[u] = a.sel[e];
+        rd[u] = a.dt[e];
         rr[u] = a.r[e];
         rv0[u] = a.v[2 * e];
         rv1[u] = a.v[2 * e + 1];
@@ -368,7 +363,6 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
         sb[u] = bf16_to_f32(rb[u]);
         ss[u] = bf16_to_f32(rs[u]);
         sd[u] = bf16_to_f32(rd[u]);
-        sd2[u] = bf16_to_f32(rd2[u]);
         sr4[u] = bf16_to_f32(rr[u]);
         sv0[u] = bf16_to_f32(rv0[u]);
         sv1[u] = bf16_to_f32(rv1[u]);
@@ -379,8 +373,7 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
         const int b = b0 + u;
         if (b < nb) {
           const bool real = hok && 16 * b + i < nt;
-          const Transition tr =
-              ABAR ? Transition{sd[u], sd2[u], sr4[u]} : cayley_gated(sd[u], sr4[u], al, om, a.c);
+          const Transition tr = cayley_gated(sd[u], sr4[u], al, om, a.c);
           const float bt = real ? sb[u] : 0.0f;
           const float fw = bt * tr.vp;
           const float wr = real ? fw * sv0[u] : 0.0f, wi = real ? fw * sv1[u] : 0.0f;
@@ -808,18 +801,18 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
 // with more segments than that run the persistent fused_fwd_onepass_kernel: a loop over segments here
 // keeps the staging's pointers live through the passes (46 to 190 scalar registers spilled), and measured
 // slower than that kernel from two rounds on (B1 H32 L65536 D64: 196-206 against 177 us).
-template <int D, bool ABAR>
+template <int D>
 __global__ __launch_bounds__(kWave* kOnePassW, D == 64 ? 2 : 1) void mf_onepass_kernel(MfArgs a) {
-  mf_segment<D, ABAR>(a, int(blockIdx.x), call_epoch(a.ob));
+  mf_segment<D>(a, int(blockIdx.x), call_epoch(a.ob));
 }
 
-template <int D, bool ABAR>
+template <int D>
 int mf_capacity(int Q) {
-  return cdssm_host::resident_capacity(reinterpret_cast<const void*>(&mf_onepass_kernel<D, ABAR>), kWave * kOnePassW,
+  return cdssm_host::resident_capacity(reinterpret_cast<const void*>(&mf_onepass_kernel<D>), kWave * kOnePassW,
                                        MfCfg<D>::lds_bytes(Q));
 }
 
-template <int D, bool ABAR>
+template <int D>
 int mf_launch(const MfmaForward& p, hipStream_t stream, hipEvent_t* ev) {
   const FwdLayout w = fwd_layout(p.B, p.L, p.H, D, p.Q);
   MfArgs a;
@@ -844,15 +837,13 @@ int mf_launch(const MfmaForward& p, hipStream_t stream, hipEvent_t* ev) {
   a.ob.grp_g = a.ob.grp_f + int64_t(p.B) * fwd_groups(w.NSEG) * p.H * D;
   a.L = p.L;
   a.H = p.H;
-  a.R = p.R;
   a.Q = p.Q;
   a.NC = w.NC;
   a.NSEG = w.NSEG;
   a.B = p.B;
   a.n_hg = (p.H + kMfHeads - 1) / kMfHeads;
   auto on = [](const void* x, uintptr_t n) { return (reinterpret_cast<uintptr_t>(x) & (n - 1)) == 0; };
-  a.wide = p.R == 1 && p.H % kMfHeads == 0 && on(p.beta, 8) && on(p.sel_c, 8) && on(p.r, 8) &&
-           (p.abar ? on(p.dt, 4) : on(p.dt, 8)) && on(p.v, 4);
+  a.wide = p.H % kMfHeads == 0 && on(p.beta, 8) && on(p.sel_c, 8) && on(p.dt, 8) && on(p.r, 8) && on(p.v, 4);
   const int64_t items = int64_t(w.NSEG) * p.B * a.n_hg;
   a.stamps = nullptr;
   if (p.stamps) {
@@ -871,7 +862,7 @@ int mf_launch(const MfmaForward& p, hipStream_t stream, hipEvent_t* ev) {
   }
   if (ev)
     for (int n = 0; n < 4; ++n) (void)hipEventRecord(ev[n], stream);
-  hipLaunchKernelGGL((mf_onepass_kernel<D, ABAR>), dim3(unsigned(items)), dim3(kWave * kOnePassW),
+  hipLaunchKernelGGL((mf_onepass_kernel<D>), dim3(unsigned(items)), dim3(kWave * kOnePassW),
                      MfCfg<D>::lds_bytes(p.Q), stream, a);
   const int st = cdssm_host::check_launch("cdssm_fused_scan_fwd/mfma");
   if (ev) (void)hipEventRecord(ev[4], stream);
@@ -880,17 +871,13 @@ int mf_launch(const MfmaForward& p, hipStream_t stream, hipEvent_t* ev) {
 
 }  // namespace
 
-bool mfma_forward_fits(int64_t B, int64_t L, int64_t H, int D, int Q, bool abar) {
+bool mfma_forward_fits(int64_t B, int64_t L, int64_t H, int D, int Q) {
   const int64_t nc = (L + Q - 1) / Q, nseg = (nc + kOnePassW - 1) / kOnePassW;
-  const int cap = D == 64 ? (abar ? mf_capacity<64, true>(Q) : mf_capacity<64, false>(Q))
-                          : (abar ? mf_capacity<128, true>(Q) : mf_capacity<128, false>(Q));
-  const int64_t items = nseg * B * ((H + kMfHeads - 1) / kMfHeads);
-  return items <= cap;
+  return nseg * B * ((H + kMfHeads - 1) / kMfHeads) <= (D == 64 ? mf_capacity<64>(Q) : mf_capacity<128>(Q));
 }
 
 int launch_mfma_forward(const MfmaForward& p, hipStream_t stream, hipEvent_t* ev) {
-  if (p.D == 64) return p.abar ? mf_launch<64, true>(p, stream, ev) : mf_launch<64, false>(p, stream, ev);
-  return p.abar ? mf_launch<128, true>(p, stream, ev) : mf_launch<128, false>(p, stream, ev);
+  return p.D == 64 ? mf_launch<64>(p, stream, ev) : mf_launch<128>(p, stream, ev);
 }
 
 int mfma_forward_status(bool clear, unsigned* out) {

@@ -1,4 +1,4 @@
-"""GPU parity of the matrix-core one-launch forward (the bf16 inference forward where one round of
+"""GPU parity of the matrix-core one-launch forward (the bf16 scan-level inference forward where one round of
 workgroups holds every segment) at the sizes where its blocks, chunks and head groups end, against the
 fp64 oracle on the same rounded inputs.
 
@@ -11,7 +11,6 @@ import pytest
 import torch
 
 from _gpu_util import DEV, ScanConfig, draw_inputs, log, oracle_fwd, rel, to_dev
-from oracle import cdssm_oracle as o
 
 pytestmark = pytest.mark.gpu
 
@@ -50,27 +49,6 @@ def test_strong_decay_runs_blocks_in_true_units(D, alpha, omega):
     y, h = run(to_dev(x))
     yr, hr = oracle_fwd(x)
     assert rel(y, yr) <= TOL_Y and rel(h, hr) <= TOL_H, (rel(y, yr), rel(h, hr))
-
-
-@pytest.mark.parametrize("N", [2, 4, 6, 16])
-def test_gate_level_rows_match_oracle(N):
-    """State rows as virtual heads: 4 consecutive ones of a wave may share a key head or not (N / 2 = 1, 2, 3, 8)."""
-    from cdssm_hip import chunkwise_delta_scan_abar
-    B, H, L, D = 2, 3, 150, 64
-    log(f"[mfma forward] gate level N={N}")
-    g = torch.Generator().manual_seed(N)
-    n = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
-    q, k = (torch.nn.functional.normalize(n(B, L, H, D), dim=-1) for _ in range(2))
-    A = torch.polar(torch.sigmoid(n(B, L, H, N // 2) + 2), n(B, L, H, N // 2))
-    x = [t.bfloat16() for t in (q, k, n(B, L, H, N), torch.sigmoid(n(B, L, H)), torch.sigmoid(n(B, L, H)),
-                                torch.view_as_real(A).flatten(-2), torch.sigmoid(n(B, L, H, N // 2)))]
-    h0 = 0.1 * n(B, H, N, D)
-    y, h = chunkwise_delta_scan_abar(*[t.to(DEV) for t in x], h0=h0.to(DEV))
-    q, k, v, beta, sel, A, vp = [t.double() for t in x]
-    Y, hr = o.ssd_chunkwise_scan(A, k, v * vp.repeat_interleave(2, dim=-1), beta, D, N, h0=h0.double(),
-                                 return_final=True)
-    yr = o.readout(Y, q, sel)
-    assert rel(y, yr) <= TOL_Y and rel(h, hr) <= 1e-6 * 4, (rel(y, yr), rel(h, hr))
 
 
 def test_misaligned_scalars_take_the_element_loads():
