@@ -11,14 +11,22 @@
 // once and a 128 KB activation many times; the library GEMMs tile them for
 // large M.  (At N = 32000, the tied head, the activation's re-reads dominate:
 // 46 us here against 18 us for the library GEMM.)  Here a workgroup owns 16
-// output columns and all M <= 64 rows: its waves split K (8 waves when K is a
+// output columns and 16, 32 or 64 rows: its waves split K (8 waves when K is a
 // multiple of 256, so that at K = 1024 each wave issues all of its loads in
 // one batch; 4 otherwise), each running v_mfma_f32_16x16x32_bf16 on operands
 // loaded straight from global memory in the instruction's layout (a 16-byte
 // load per lane per fragment: rows of X, rows of W), and the waves' partial
-// tiles are summed in a fixed order through LDS.
-// So W streams from HBM once with 16-byte loads, X is served by the L2, and a
-// call launches ceil(N / 16) workgroups.
+// tiles are summed in a fixed order through LDS.  The order of every sum is
+// the same for any number of rows per workgroup.
+//
+// A call is one latency chain: its weight rows, its activation rows, the sum.
+// What bounds it is how many loads one CU has to issue and return, so the rows
+// are split over the CUs as far as one round of workgroups takes them
+// (kOneRound).  Measured on MI355X at M = 64, K = 1024, us per call back to
+// back, for 16 / 32 / 64 rows per workgroup: N = 1024 4.5 / 5.2 / 7.0,
+// N = 1552 6.2 / 5.3 / 6.9, N = 2048 6.2 / 5.5 / 7.3, N = 3104 9.7 / 8.6 / 7.9;
+// with the norm at N = 1024 5.2 / 6.0 / 8.0, N = 3104 10.9 / 8.9 / 8.9.  At
+// M = 16, K = 2048, N = 4096 7.5 / 7.7 / 9.0.  (Always 64 rows before.)
 //
 // Fragment layouts of v_mfma_f32_16x16x32_bf16 (checked on MI355X):
 //   A (16 x 32): lane l holds row l % 16, k = 8 (l / 16) .. + 8
@@ -36,6 +44,9 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kCols = 16;   // output columns per workgroup
 constexpr int kMaxRows = 64;
+// Workgroups that count as one round: one per CU (256), and an eighth of the CUs may hold a second one
+// (N = 1136, M = 64: 284 workgroups of 16 rows 6.0 us, 142 of 32 rows 6.25; N = 1552: 388 of 16 6.2, 194 of 32 5.3).
+constexpr int64_t kOneRound = 288;
 constexpr int kUnroll = 4;  // k-steps (of 32) whose loads are issued together
 
 __device__ __forceinline__ uint4 ld16(const uint16_t* p) { return *reinterpret_cast<const uint4*>(p); }
@@ -60,49 +71,56 @@ __device__ __forceinline__ float sumsq_frag(uint4 a, float s) {
   return s;
 }
 
-template <bool NORM, int kWaves>
+// 16 * MT rows by 16 columns per workgroup.
+template <bool NORM, int kWaves, int MT>
 __global__ __launch_bounds__(kWave * kWaves) void skinny_gemm_kernel(
     const uint16_t* __restrict__ X, int64_t ldx, const uint16_t* __restrict__ W, int64_t ldw,
     const uint16_t* __restrict__ bias, const uint16_t* __restrict__ R, int64_t ldr,
     const uint16_t* __restrict__ wnorm, float eps, uint16_t* __restrict__ Y, int64_t ldy, int M, int N, int K) {
-  __shared__ f32x4_t part[kWaves][kMaxRows / 16][kWave];  // 4 KB per wave: its partial tiles
-  __shared__ float ssq[kWaves][kMaxRows];                  // each wave's partial row sums of squares
+  __shared__ f32x4_t part[kWaves][MT][kWave];  // 1 KB per wave and row tile: its partial tiles
+  __shared__ float ssq[kWaves][16 * MT];       // each wave's partial row sums of squares
   const int wave = int(threadIdx.x) / kWave;
   const int lane = int(threadIdx.x) % kWave;
   const int col = lane % 16, kq = lane / 16;
-  const int n0 = int(blockIdx.x) * kCols;
+  // the row groups of a column tile lie 8 workgroups apart (one XCD under the round-robin placement), so the
+  // tile's weight rows come from HBM once and from that XCD's L2 for the others
+  const int n_nt = (N + kCols - 1) / kCols, n_mg = (M + 16 * MT - 1) / (16 * MT);
+  const int grp = int(blockIdx.x) / (8 * n_mg), loc = int(blockIdx.x) - grp * 8 * n_mg;
+  const int width = min(8, n_nt - 8 * grp);
+  const int mg = loc / width;
+  const int n0 = (8 * grp + loc - mg * width) * kCols, m0 = mg * 16 * MT;
   const int n = min(n0 + col, N - 1);  // loads clamped into the matrix; stores masked
   const int kw = K / kWaves;
   const int kb = wave * kw;
   const uint16_t* wrow = W + int64_t(n) * ldw + kb + 8 * kq;
-  const uint16_t* xrow[kMaxRows / 16];
+  const uint16_t* xrow[MT];
 #pragma unroll
-  for (int mt = 0; mt < kMaxRows / 16; ++mt) xrow[mt] = X + int64_t(min(mt * 16 + col, M - 1)) * ldx + kb + 8 * kq;
+  for (int mt = 0; mt < MT; ++mt) xrow[mt] = X + int64_t(min(m0 + mt * 16 + col, M - 1)) * ldx + kb + 8 * kq;
   const uint16_t* nrow = NORM ? wnorm + kb + 8 * kq : nullptr;
 
-  f32x4_t acc[kMaxRows / 16];
-  float sq[kMaxRows / 16];
+  f32x4_t acc[MT];
+  float sq[MT];
 #pragma unroll
-  for (int mt = 0; mt < kMaxRows / 16; ++mt) {
+  for (int mt = 0; mt < MT; ++mt) {
     acc[mt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     sq[mt] = 0.0f;
   }
   // U k-steps of 32 from k: every load first, then the products
   const auto steps = [&](int k, auto uc) {
     constexpr int U = decltype(uc)::value;
-    uint4 b[U], a[U][kMaxRows / 16], g[U];
+    uint4 b[U], a[U][MT], g[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       b[u] = ld16(wrow + k + 32 * u);
 #pragma unroll
-      for (int mt = 0; mt < kMaxRows / 16; ++mt) a[u][mt] = ld16(xrow[mt] + k + 32 * u);
+      for (int mt = 0; mt < MT; ++mt) a[u][mt] = ld16(xrow[mt] + k + 32 * u);
       if constexpr (NORM) g[u] = ld16(nrow + k + 32 * u);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const bf16x8_t bv = __builtin_bit_cast(bf16x8_t, b[u]);
 #pragma unroll
-      for (int mt = 0; mt < kMaxRows / 16; ++mt) {
+      for (int mt = 0; mt < MT; ++mt) {
         uint4 av = a[u][mt];
         if constexpr (NORM) {
           sq[mt] = sumsq_frag(av, sq[mt]);
@@ -117,11 +135,11 @@ __global__ __launch_bounds__(kWave * kWaves) void skinny_gemm_kernel(
   for (; k + 32 * kUnroll <= kw; k += 32 * kUnroll) steps(k, std::integral_constant<int, kUnroll>{});
   for (; k < kw; k += 32) steps(k, std::integral_constant<int, 1>{});
 #pragma unroll
-  for (int mt = 0; mt < kMaxRows / 16; ++mt) part[wave][mt][lane] = acc[mt];
+  for (int mt = 0; mt < MT; ++mt) part[wave][mt][lane] = acc[mt];
   if constexpr (NORM) {
     // the lanes of a row (col) over kq: lanes col, col + 16, col + 32, col + 48
 #pragma unroll
-    for (int mt = 0; mt < kMaxRows / 16; ++mt) {
+    for (int mt = 0; mt < MT; ++mt) {
       float s = sq[mt];
       s += __shfl_xor(s, 16, kWave);
       s += __shfl_xor(s, 32, kWave);
@@ -130,8 +148,8 @@ __global__ __launch_bounds__(kWave * kWaves) void skinny_gemm_kernel(
   }
   __syncthreads();
 
-  // wave w < 4 finishes row tile w: the partials in wave order, then the epilogue
-  if (wave >= kMaxRows / 16) return;
+  // wave w < MT finishes row tile w: the partials in wave order, then the epilogue
+  if (wave >= MT) return;
   const int mt = wave;
   f32x4_t c = part[0][mt][lane];
 #pragma unroll
@@ -147,13 +165,13 @@ __global__ __launch_bounds__(kWave * kWaves) void skinny_gemm_kernel(
   const float bv = bias ? bf16_to_f32(bias[nn]) : 0.0f;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const int m = mt * 16 + 4 * kq + i;
+    const int ml = mt * 16 + 4 * kq + i, m = m0 + ml;
     if (m < M) {
       float y = c[i];
       if constexpr (NORM) {
         float s = 0.0f;
 #pragma unroll
-        for (int w = 0; w < kWaves; ++w) s += ssq[w][m];
+        for (int w = 0; w < kWaves; ++w) s += ssq[w][ml];
         s /= float(K);
         y *= __builtin_amdgcn_rsqf(s + eps);
       }
@@ -198,25 +216,30 @@ extern "C" int cdssm_skinny_gemm(int dtype, const void* X, int64_t ldx, const vo
                           "leading dimensions cover the rows");
     return CDSSM_EINVAL;
   }
-  const bool eight = K % 256 == 0;  // 8 waves of K / 8 (a multiple of 32) each
-  const dim3 grid(unsigned((N + sg::kCols - 1) / sg::kCols)), block(kWave * (eight ? 8 : 4));
   const auto* x = static_cast<const uint16_t*>(X);
   const auto* w = static_cast<const uint16_t*>(W);
   const auto* b = static_cast<const uint16_t*>(bias);
   const auto* r = static_cast<const uint16_t*>(R);
   const auto* g = static_cast<const uint16_t*>(wnorm);
   auto* y = static_cast<uint16_t*>(Y);
-  if (wnorm && eight)
-    hipLaunchKernelGGL((sg::skinny_gemm_kernel<true, 8>), grid, block, 0, stream, x, ldx, w, ldw, b, r, ldr, g, eps,
-                       y, ldy, int(M), int(N), int(K));
-  else if (wnorm)
-    hipLaunchKernelGGL((sg::skinny_gemm_kernel<true, 4>), grid, block, 0, stream, x, ldx, w, ldw, b, r, ldr, g, eps,
-                       y, ldy, int(M), int(N), int(K));
-  else if (eight)
-    hipLaunchKernelGGL((sg::skinny_gemm_kernel<false, 8>), grid, block, 0, stream, x, ldx, w, ldw, b, r, ldr, g,
-                       eps, y, ldy, int(M), int(N), int(K));
+  auto go = [&](auto norm, auto waves, auto mt) {
+    constexpr int kW = decltype(waves)::value, MT = decltype(mt)::value;
+    const dim3 grid(unsigned((N + sg::kCols - 1) / sg::kCols * ((M + 16 * MT - 1) / (16 * MT)))), block(kWave * kW);
+    hipLaunchKernelGGL((sg::skinny_gemm_kernel<decltype(norm)::value, kW, MT>), grid, block, 0, stream, x, ldx, w,
+                       ldw, b, r, ldr, g, eps, y, ldy, int(M), int(N), int(K));
+  };
+  using W8 = std::integral_constant<int, 8>;  // K a multiple of 256: K / 8 (a multiple of 32) per wave
+  using W4 = std::integral_constant<int, 4>;
+  auto rows = [&](auto norm, auto waves) {
+    const int64_t nt = (N + sg::kCols - 1) / sg::kCols, mt = (M + 15) / 16;
+    const int64_t cap = sg::kOneRound;
+    if (nt * mt <= cap) return go(norm, waves, std::integral_constant<int, 1>{});
+    if (nt * ((mt + 1) / 2) <= cap) return go(norm, waves, std::integral_constant<int, 2>{});
+    go(norm, waves, std::integral_constant<int, sg::kMaxRows / 16>{});
+  };
+  if (K % 256 == 0)
+    wnorm ? rows(std::true_type{}, W8{}) : rows(std::false_type{}, W8{});
   else
-    hipLaunchKernelGGL((sg::skinny_gemm_kernel<false, 4>), grid, block, 0, stream, x, ldx, w, ldw, b, r, ldr, g,
-                       eps, y, ldy, int(M), int(N), int(K));
+    wnorm ? rows(std::true_type{}, W4{}) : rows(std::false_type{}, W4{});
   return cdssm_host::check_launch("cdssm_skinny_gemm");
 }

@@ -85,3 +85,34 @@ def test_skinny_gemm_strided_rows_and_graph_replay():
         torch.cuda.synchronize()
         assert torch.equal(y_g.cpu(), ref.cpu()), seed
     log("[skinny gemm] strided rows, graph replays equal eager calls")
+
+
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("M,N", [
+    (64, 1152), (64, 1153), (64, 2304), (64, 2305),  # 16 | 32 and 32 | 64 rows per workgroup, M = 64
+    (48, 1536), (48, 1537), (33, 2304), (33, 2320),  # three row groups of 16, the last one of a single row
+    (17, 2304), (17, 2305), (17, 4609),              # two groups of 16, then one of 32 (the third tile unused)
+    (16, 4608), (1, 4609), (64, 7), (17, 127),       # one group; fewer column tiles than XCDs
+])
+def test_rows_per_workgroup_leave_the_sums_alone(M, N, norm):
+    """16, 32 or 64 rows go to a workgroup by M and N.  The order of every sum is the same for all of them, so
+    each row equals, bit for bit, the product of that row alone; that one is within the rounding of its bf16
+    result (2^-8 relative to the largest output) and, with the norm, of its operand (2^-8 again) of a 64-bit
+    product of the same operands."""
+    from cdssm_hip.lm import skinny_linear
+    K = 256
+    g = torch.Generator().manual_seed(M + N)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16).to(DEV)
+    w = (torch.randn(N, K, generator=g) / 16.0).to(torch.bfloat16).to(DEV)
+    bias = torch.randn(N, generator=g).to(torch.bfloat16).to(DEV)
+    res = torch.randn(M, N, generator=g).to(torch.bfloat16).to(DEV)
+    nw = (1.0 + 0.1 * torch.randn(K, generator=g)).to(torch.bfloat16).to(DEV) if norm else None
+    y = skinny_linear(x, w, bias, res, nw, 1e-5)
+    for m in sorted({0, 15, 16, 31, 32, M - 1} & set(range(M))):
+        one = skinny_linear(x[m:m + 1], w, bias, res[m:m + 1], nw, 1e-5)
+        assert torch.equal(y[m:m + 1], one), f"row {m}"
+    x64 = x.double()
+    if norm:
+        x64 = x64 * torch.rsqrt(x64.pow(2).mean(-1, keepdim=True) + 1e-5) * nw.double()
+    ref = (x64 @ w.double().t() + bias.double() + res.double()).cpu()
+    assert rel(y.double().cpu(), ref) <= (2 if norm else 1) * 2.0 ** -8 + 1e-5
