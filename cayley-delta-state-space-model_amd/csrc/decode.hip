@@ -236,19 +236,47 @@ __device__ __forceinline__ void decode_token_wave(
   const typename T::raw* grow = gq + int64_t(bi) * a.gq_stride;
   const typename T::raw* prow = proj + int64_t(bi) * a.proj_stride;
 
+  // Every load of the step goes out here, the token's scalars first: they come back first, and the dynamics
+  // run while the rows and the state are on their way.
+  typename T::raw gr[N + 5];
+#pragma unroll
+  for (int j = 0; j < N + 5; ++j) gr[j] = grow[int64_t(j) * H + hl];
+  const int64_t l = *a.l_dev;
+  const float rope = a.rope[hl], lds = a.lds[hl], scale = a.scale[0];
+  const typename T::raw* vp = prow + a.v_off + 2 * hl;
+  const typename T::raw* fp = v_first ? v_first + 2 * bh : vp;  // without a layer 0 value: read, not used
+  const typename T::raw v_raw[2] = {vp[0], vp[1]}, f_raw[2] = {fp[0], fp[1]}, w_raw = *(v_first ? vgate + hl : vp);
+  const float2 g = gam[bh];
+  const int jpos = pos[bh];
+  RowVec<T, DPL> kv, qv;
+  kv.load(prow + a.k_off + hl * D + sub * DPL);
+  qv.load(grow + (N + 5) * H + hl * D + sub * DPL);
+  float* st = state + bh * 6 * D + sub * DPL;
+  float zr[DPL], zi[DPL], cr[DPL], ci[DPL];
+#pragma unroll
+  for (int j = 0; j < DPL; j += 4) {
+    const float4 a0 = *reinterpret_cast<const float4*>(st + j);
+    const float4 a1 = *reinterpret_cast<const float4*>(st + D + j);
+    const float4 a2 = *reinterpret_cast<const float4*>(st + 2 * D + j);
+    const float4 a3 = *reinterpret_cast<const float4*>(st + 3 * D + j);
+    zr[j] = a0.x; zr[j + 1] = a0.y; zr[j + 2] = a0.z; zr[j + 3] = a0.w;
+    zi[j] = a1.x; zi[j + 1] = a1.y; zi[j + 2] = a1.z; zi[j + 3] = a1.w;
+    cr[j] = a2.x; cr[j + 1] = a2.y; cr[j + 2] = a2.z; cr[j + 3] = a2.w;
+    ci[j] = a3.x; ci[j + 1] = a3.y; ci[j + 2] = a3.z; ci[j + 3] = a3.w;
+  }
+
   // dynamics at the token's position, rounded as DynamicsFusedFn stores them
-  const float pp = float(*a.l_dev) * a.rope[hl];
-  const gates::GateToken gt = gates::gate_token<T>(grow + hl, H, N, a.lds[hl], pp, a.kc);
-  const Transition tr0 = gates::gate_pair<T>(grow + hl, H, N, 0, pp, gt, a.kc);
+  const float pp = float(l) * rope;
+  const gates::GateToken gt = gates::gate_token<T>(gr, 1, N, lds, pp, a.kc);
+  const Transition tr0 = gates::gate_pair<T>(gr, 1, N, 0, pp, gt, a.kc);
   const Transition tr{round_to<T>(tr0.ar), round_to<T>(tr0.ai), round_to<T>(tr0.vp)};
   const float bb = round_to<T>(gt.beta), sc = round_to<T>(gt.selc);
 
   // V (B, H, 2): the in_proj's, or the value-residual lerp with layer 0's
-  float v0 = T::load(prow + a.v_off + 2 * hl), v1 = T::load(prow + a.v_off + 2 * hl + 1);
+  float v0 = T::load(&v_raw[0]), v1 = T::load(&v_raw[1]);
   if (v_first) {
+    const float w = T::load(&w_raw), s0 = T::load(&f_raw[0]), s1 = T::load(&f_raw[1]);
     // torch.lerp(start, end, w): start + w (end - start) for w < 0.5, else end - (end - start)(1 - w)
-    const float w = T::load(vgate + hl);
-    const float s0 = T::load(v_first + 2 * bh), s1 = T::load(v_first + 2 * bh + 1);
     v0 = round_to<T>(w < 0.5f ? fmaf(w, v0 - s0, s0) : v0 - (v0 - s0) * (1.0f - w));
     v1 = round_to<T>(w < 0.5f ? fmaf(w, v1 - s1, s1) : v1 - (v1 - s1) * (1.0f - w));
   }
@@ -256,13 +284,8 @@ __device__ __forceinline__ void decode_token_wave(
 
   // K, Q normalised (the same lane split and summation order as normalize_qk_kernel)
   float kk[DPL], qq[DPL];
-  {
-    RowVec<T, DPL> kv, qv;
-    kv.load(prow + a.k_off + hl * D + sub * DPL);
-    qv.load(grow + (N + 5) * H + hl * D + sub * DPL);
-    kv.unpack(kk);
-    qv.unpack(qq);
-  }
+  kv.unpack(kk);
+  qv.unpack(qq);
   float sk = 0.0f, sq = 0.0f;
 #pragma unroll
   for (int j = 0; j < DPL; ++j) {
@@ -282,21 +305,6 @@ __device__ __forceinline__ void decode_token_wave(
   qkd = group_sum<LPH>(qkd);
 
   // the scan's decode step (decode_step_kernel's arithmetic)
-  float* st = state + bh * 6 * D + sub * DPL;
-  float zr[DPL], zi[DPL], cr[DPL], ci[DPL];
-#pragma unroll
-  for (int j = 0; j < DPL; j += 4) {
-    const float4 a0 = *reinterpret_cast<const float4*>(st + j);
-    const float4 a1 = *reinterpret_cast<const float4*>(st + D + j);
-    const float4 a2 = *reinterpret_cast<const float4*>(st + 2 * D + j);
-    const float4 a3 = *reinterpret_cast<const float4*>(st + 3 * D + j);
-    zr[j] = a0.x; zr[j + 1] = a0.y; zr[j + 2] = a0.z; zr[j + 3] = a0.w;
-    zi[j] = a1.x; zi[j + 1] = a1.y; zi[j + 2] = a1.z; zi[j + 3] = a1.w;
-    cr[j] = a2.x; cr[j + 1] = a2.y; cr[j + 2] = a2.z; cr[j + 3] = a2.w;
-    ci[j] = a3.x; ci[j + 1] = a3.y; ci[j + 2] = a3.z; ci[j + 3] = a3.w;
-  }
-  const float2 g = gam[bh];
-  const int jpos = pos[bh];
   float pzr = 0.0f, pzi = 0.0f, pcr = 0.0f, pci = 0.0f, cqr = 0.0f, cqi = 0.0f;
 #pragma unroll
   for (int j = 0; j < DPL; ++j) {
@@ -334,7 +342,7 @@ __device__ __forceinline__ void decode_token_wave(
   if (!hok) return;  // nothing below reduces across lanes
   if (sub == 0) {
     // the shortcut through the readout (shortcut_kernel's arithmetic)
-    const float c = a.scale[0] * qkd * qkd * sc * tr.vp;
+    const float c = scale * qkd * qkd * sc * tr.vp;
     if (rs) {
       rs[2 * hl] = round_to<T>(yr + c * v0);
       rs[2 * hl + 1] = round_to<T>(yi + c * v1);
@@ -394,11 +402,13 @@ __global__ __launch_bounds__(kWave) void decode_token_kernel(
                                proj, v_first, vgate, state, gam, pos, ret, nullptr, v_out, a);
 }
 
+constexpr int kTailWaves = 8;  // the decode tail's waves beside those of the token step
+
 // The block's decode tail in one launch (block.py:169-225 after the gate / Q
 // projection): one workgroup per batch row, a wave per group of HPW heads
 // running decode_token_wave into LDS, then the row's readout projection and
 // GroupNorm + gate step (lm::gn_row_step).  position[0] is the layer's decode
-// position and position[1] an arrival count: every workgroup arrives once it
+// position and position[1] an arrival count: every workgroup arrives after it
 // has read the position, and the last to arrive advances it and clears the
 // count (so the next launch, and a replayed graph, find it zero).
 struct DecodeTailArgs {
@@ -412,6 +422,12 @@ struct DecodeTailArgs {
   unsigned long long* arrive;  // position + 1
 };
 
+// One workgroup is one latency chain (64 of them at a batch of 64 rows leave three CUs in four idle), and
+// memory answers in about a microsecond: what it costs is the number of loads that wait for one another.  So
+// the token waves request their rows and their state before they compute the token's dynamics, and 8 more
+// waves, which have no part in the token step, meanwhile hold everything the epilogue reads in registers
+// (lm::RowPrefetch).  B 64, H 16, D 64, C 1024, bf16 on MI355X: 14.9 -> 9.1 us, of which 4.2 the token step
+// and 3.1 the epilogue; the arrival at the end and relaxed instead of acquire-release in the middle.
 template <typename T, int D, int LPH, typename P>
 __global__ __launch_bounds__(1024) void decode_tail_kernel(
     const typename T::raw* __restrict__ gq, const typename T::raw* __restrict__ proj,
@@ -420,30 +436,50 @@ __global__ __launch_bounds__(1024) void decode_tail_kernel(
     DecodeTokenArgs a, DecodeTailArgs t) {
   using raw = typename T::raw;
   constexpr int HPW = kWave / LPH;
-  extern __shared__ float tail_lds[];
+  extern __shared__ __align__(16) float tail_lds[];
   const int kr = 2 * a.H;
   float* rs = tail_lds;                                                  // the row's retrieved values (kr)
   float2* gst = reinterpret_cast<float2*>(tail_lds + ((kr + 1) & ~1));  // (mean, rstd) per group
-  float* ys = reinterpret_cast<float*>(gst + t.G);                       // the row's y (C)
+  float* ys = reinterpret_cast<float*>(gst + t.G);                       // the row's y (lm::ys_at)
   const int bi = int(blockIdx.x);
-  const int wv = int(threadIdx.x) / kWave;
-  // the first n_hg waves run the token step; the whole workgroup (at least 8 waves) the epilogue
-  if (wv < a.n_hg)
+  const int wv = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / kWave);
+  const lm::RowArgs<T, P> row{static_cast<const raw*>(t.wr), kr, t.gsum, static_cast<const typename P::raw*>(t.gamma),
+                              static_cast<const typename P::raw*>(t.beta), static_cast<const raw*>(t.z), t.z_bs,
+                              static_cast<const raw*>(t.xc), static_cast<const raw*>(t.Dp), static_cast<raw*>(t.out),
+                              t.C, t.G, t.eps};
+  auto token = [&] {
     decode_token_wave<T, D, LPH>(bi, wv * HPW, int(threadIdx.x) % kWave, gq, proj, v_first, vgate, state, gam, pos,
                                  nullptr, rs, v_out, a);
-  __syncthreads();  // every wave has read the position and written its heads' retrieved values
+  };
+  // the first n_hg waves run the token step, the others the epilogue; where that leaves fewer than kTailWaves,
+  // the whole workgroup runs both.  The branches are taken by whole waves, and each passes the same three
+  // barriers: after the first, every wave has read the position and written its heads' retrieved values.
+  if (int(blockDim.x) / kWave < a.n_hg + kTailWaves) {
+    if (wv < a.n_hg) token();
+    __syncthreads();
+    lm::gn_row_step<T, P, false>(bi, nullptr, rs, row, gst, ys, int(threadIdx.x), int(blockDim.x), {});
+  } else if (wv < a.n_hg) {
+    token();
+    __syncthreads();
+    __syncthreads();
+    __syncthreads();
+  } else {
+    const int tid = int(threadIdx.x) - a.n_hg * kWave, nthr = int(blockDim.x) - a.n_hg * kWave;
+    lm::RowPrefetch<T, P> pf;
+    pf.load(bi, row, tid, nthr);
+    __syncthreads();
+    lm::gn_row_step<T, P, true>(bi, nullptr, rs, row, gst, ys, tid, nthr, pf);
+  }
+  // The arrival comes last and relaxed: every read of the position has returned (its value went into rs), and
+  // the position is read again only by later kernels.
   if (threadIdx.x == 0) {
-    const unsigned long long n = __hip_atomic_fetch_add(t.arrive, 1ull, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned long long n = __hip_atomic_fetch_add(t.arrive, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (n + 1 == gridDim.x) {
       __hip_atomic_store(t.arrive, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       int64_t* position = const_cast<int64_t*>(a.l_dev);
       position[0] += 1;
     }
   }
-  lm::gn_row_step<T, P>(bi, nullptr, rs, static_cast<const raw*>(t.wr), kr, t.gsum,
-                        static_cast<const typename P::raw*>(t.gamma), static_cast<const typename P::raw*>(t.beta),
-                        static_cast<const raw*>(t.z), t.z_bs, static_cast<const raw*>(t.xc),
-                        static_cast<const raw*>(t.Dp), static_cast<raw*>(t.out), t.C, t.G, t.eps, gst, ys);
 }
 
 // state = (0, h, h) per (b, h) (h = 0 if null), g = 1, j = 0: the decode state
@@ -716,14 +752,15 @@ extern "C" int cdssm_decode_block_tail(int dtype, int param_dtype, const void* g
   t.G = int(G);
   t.eps = eps;
   t.arrive = reinterpret_cast<unsigned long long*>(position + 1);
-  const size_t lds = size_t((2 * H + 1) / 2 * 2 + 2 * G + C) * sizeof(float);
+  const int y_floats = lm::ys_at(int(C), lm::ys_shift(int(C), int(G)));
+  const size_t lds = size_t((2 * H + 1) / 2 * 2 + 2 * G + y_floats) * sizeof(float);
   auto go = [&](auto tt, auto pt, auto dc, auto lc) {
     using T = decltype(tt);
     using P = decltype(pt);
     using raw = typename T::raw;
     constexpr int DD = decltype(dc)::value, LP = decltype(lc)::value, HPW = kWave / LP;
     a.n_hg = int((H + HPW - 1) / HPW);
-    const unsigned threads = unsigned(kWave * std::max(a.n_hg, 8));
+    const unsigned threads = unsigned(kWave * (a.n_hg <= 16 - kTailWaves ? a.n_hg + kTailWaves : a.n_hg));
     hipLaunchKernelGGL((decode_tail_kernel<T, DD, LP, P>), dim3(unsigned(B)), dim3(threads), lds,
                        stream, static_cast<const raw*>(gq), static_cast<const raw*>(proj),
                        static_cast<const raw*>(v_first), static_cast<const raw*>(vgate), state,

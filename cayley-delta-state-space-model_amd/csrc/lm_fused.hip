@@ -667,7 +667,7 @@ __global__ __launch_bounds__(256) void gn_gate_step_kernel(const typename T::raw
   // (mean, rstd) per group; with ret, the row's y (C values) and retrieved row (kr values) after them
   extern __shared__ float2 gst[];
   float* ys = reinterpret_cast<float*>(gst + G);
-  float* rs = ys + C;
+  float* rs = ys + ys_at(C, ys_shift(C, G));
   // the layer's decode position advances with its last per-token kernel
   if (position && blockIdx.x == 0 && threadIdx.x == 0) position[0] += 1;
   const int b = blockIdx.x;
@@ -676,7 +676,8 @@ __global__ __launch_bounds__(256) void gn_gate_step_kernel(const typename T::raw
     for (int j = threadIdx.x; j < kr; j += blockDim.x) rs[j] = T::load(rr + j);
     __syncthreads();
   }
-  gn_row_step<T, P>(b, y, ret ? rs : nullptr, wr, kr, gsum, gamma, beta, z, z_bs, xc, Dp, out, C, G, eps, gst, ys);
+  const RowArgs<T, P> row{wr, kr, gsum, gamma, beta, z, z_bs, xc, Dp, out, C, G, eps};
+  gn_row_step<T, P, false>(b, y, ret ? rs : nullptr, row, gst, ys, int(threadIdx.x), int(blockDim.x), {});
 }
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -1504,7 +1505,7 @@ static int gn_step(const char* op, int dtype, int param_dtype, const void* y, co
     auto go = [&](auto pt) {
       using P = decltype(pt);
       using praw = typename P::raw;
-      const size_t lds = size_t(G) * sizeof(float2) + (ret ? size_t(C + kr) * sizeof(float) : 0);
+      const size_t lds = size_t(G) * sizeof(float2) + (ret ? size_t(ys_at(int(C), ys_shift(int(C), int(G))) + kr) * sizeof(float) : 0);
       hipLaunchKernelGGL((gn_gate_step_kernel<T, P>), dim3(unsigned(B)), dim3(256), lds, stream,
                          static_cast<const raw*>(y), static_cast<const raw*>(ret), static_cast<const raw*>(wr),
                          int(kr), reinterpret_cast<float4*>(gsum),

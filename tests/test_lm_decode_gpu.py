@@ -282,6 +282,48 @@ def test_fused_tail_matches_token_kernel_and_separate_epilogue(dtype, d_inner):
             assert torch.equal(c1["scan"].state, c2["scan"].state)
 
 
+@pytest.mark.parametrize("dtype,head_dim,H", [
+    (torch.bfloat16, 64, 2),    # fewer channels than threads; 8-byte weight rows: read element by element
+    (torch.bfloat16, 64, 20),   # the last token wave half empty; three channels on some threads: not held
+    (torch.bfloat16, 64, 32),   # 16-byte rows, four channels per thread: more weights than a thread holds
+    (torch.bfloat16, 64, 64),   # the largest that leaves 8 waves beside the token's
+    (torch.bfloat16, 64, 72),   # one token wave more: the workgroup runs both parts
+    (torch.bfloat16, 128, 4),
+    (torch.float32, 64, 4),
+    (torch.float32, 64, 36),    # 9 token waves
+    (torch.float32, 128, 18),
+])
+def test_tail_waves_and_held_rows_at_their_edges(dtype, head_dim, H):
+    """The tail's epilogue runs on waves of its own where the token step leaves 8 of 16, on rows held in registers
+    where they fit.  Same arithmetic in the same order as the separate kernels: equal bits."""
+    from cdssm_hip.lm import CDSSMBlock, CDSSMConfig, CDSSMLMHeadModel, _clone_cache
+    torch.manual_seed(H)
+    cfg = CDSSMConfig(d_model=128, n_layers=2, context_length=128, vocab_size=97, state_dim=2, d_inner=H * head_dim,
+                      head_dim=head_dim)
+    m = CDSSMLMHeadModel(cfg)
+    with torch.no_grad():
+        for blk in m.blocks:
+            blk.v_residual_gate.normal_(std=1.0)
+            blk.shortcut_scale.fill_(0.3)
+            blk.D.normal_(std=0.1)
+    m = m.to(dtype).to(DEV).eval()
+    ids = torch.randint(0, cfg.vocab_size, (3, 12), generator=torch.Generator().manual_seed(H)).to(DEV)
+    with torch.no_grad():
+        _, ca = m.prefill(ids[:, :10])
+        cb = [_clone_cache(c) for c in ca]
+        try:
+            for t in (10, 11):
+                CDSSMBlock.fused_tail = True
+                la = m.decode_step(ids[:, t], ca)
+                CDSSMBlock.fused_tail = False
+                assert torch.equal(la, m.decode_step(ids[:, t], cb))
+        finally:
+            CDSSMBlock.fused_tail = True
+    for c1, c2 in zip(ca, cb):
+        assert torch.equal(c1["l"], c2["l"]) and c1["l"].tolist() == [12, 0]
+        assert torch.equal(c1["gsum"], c2["gsum"]) and torch.equal(c1["scan"].state, c2["scan"].state)
+
+
 def test_config4_decode_24_layers_batch_64():
     """Config 4's decode: 24 layers, d_model 1024, 16 heads x 64, vocab 32000, bf16, B = 64 from a
     2048-token prefill.  Each step is finite; the graph-captured step equals the eager step on every
