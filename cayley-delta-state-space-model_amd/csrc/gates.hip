@@ -21,6 +21,8 @@
 // normalize fwd/bwd (NormalizeKQFn, ops.py:84-97; normalize_kq.cu:75-79,
 //   :143-163): x_hat = x rsqrt(sum x^2 + 1e-6); g_in = (g - x_hat <g, x_hat>) rsqrt(...).
 //   Any head_dim D <= 256 (the reference kernel is correct only for D = 64).
+#include <type_traits>
+
 #include "gate_math.hpp"
 
 namespace cdssm {
@@ -39,58 +41,138 @@ __device__ __forceinline__ bool gate_idx(int64_t tid, int L, int H, int64_t tota
   return true;
 }
 
-template <typename T>
+// n elements between memory and registers in accesses of up to 16 bytes (p aligned to min(16, n elements)).
+template <int BYTES>
+struct WideOf {
+  using type = uint4;
+};
+template <>
+struct WideOf<8> {
+  using type = uint2;
+};
+template <>
+struct WideOf<4> {
+  using type = uint32_t;
+};
+template <>
+struct WideOf<2> {
+  using type = uint16_t;
+};
+template <typename R, int n>
+struct WideRow {
+  using W = typename WideOf<(n * int(sizeof(R)) < 16 ? n * int(sizeof(R)) : 16)>::type;
+  static constexpr int M = n * int(sizeof(R)) / int(sizeof(W));
+  union {
+    W w[M];
+    R e[n];
+  };
+  __device__ __forceinline__ void load(const R* p) {
+#pragma unroll
+    for (int i = 0; i < M; ++i) w[i] = reinterpret_cast<const W*>(p)[i];
+  }
+  __device__ __forceinline__ void store(R* p) const {
+#pragma unroll
+    for (int i = 0; i < M; ++i) reinterpret_cast<W*>(p)[i] = w[i];
+  }
+};
+
+// NH = N / 2 pairs: for the usual state sizes a constant, with the token's gates requested before any is used
+// and its A_bar and vp rows stored whole; 0 for every other N, a pair's loads after the previous pair's
+// arithmetic and 2-byte stores.  B 4, L 2048, H 24, N 16, bf16 on MI355X: 18.9 -> 14.2 us; B 8, L 2048, H 16,
+// N 2: 8.0 -> 7.2 us.
+template <typename T, int NH>
 __global__ __launch_bounds__(256) void dynamics_fwd_kernel(
     const typename T::raw* __restrict__ gate, const float* __restrict__ log_dt_scale,
     const float* __restrict__ rope, typename T::raw* __restrict__ A_out, typename T::raw* __restrict__ vp_out,
     typename T::raw* __restrict__ beta_out, typename T::raw* __restrict__ selc_out, float gating_c,
-    float omega_thresh, float adt_delta, float adt_smooth, float adt_eps, int L, int H, int N,
+    float omega_thresh, float adt_delta, float adt_smooth, float adt_eps, int L, int H, int Nrt,
     int64_t total, int64_t l0, const int64_t* __restrict__ l0_dev) {
   GateIdx g;
   if (!gate_idx(int64_t(blockIdx.x) * blockDim.x + threadIdx.x, L, H, total, g)) return;
+  const int N = NH > 0 ? 2 * NH : Nrt;
   const int Nh = N / 2, G = N + 5;
   const typename T::raw* row = gate + g.bl * int64_t(G) * H + g.h;
-  const float freq = rope[g.h];
-  const float pos = float(g.l + l0 + (l0_dev ? *l0_dev : 0)) * freq;  // sequence position
-  const GateConsts kc{gating_c, omega_thresh, adt_delta, adt_smooth, adt_eps};
-  const GateToken gt = gate_token<T>(row, H, N, log_dt_scale[g.h], pos, kc);
   const int64_t o = g.bl * H + g.h;
-  for (int j = 0; j < Nh; ++j) {
-    const Transition tr = gate_pair<T>(row, H, N, j, pos, gt, kc);
-    T::store(A_out + o * N + 2 * j, tr.ar);
-    T::store(A_out + o * N + 2 * j + 1, tr.ai);
-    T::store(vp_out + o * Nh + j, tr.vp);
+  const GateConsts kc{gating_c, omega_thresh, adt_delta, adt_smooth, adt_eps};
+  if constexpr (NH > 0) {
+    typename T::raw gr[2 * NH + 5];
+#pragma unroll
+    for (int s = 0; s < 2 * NH + 5; ++s) gr[s] = row[int64_t(s) * H];
+    const float pos = float(g.l + l0 + (l0_dev ? *l0_dev : 0)) * rope[g.h];  // sequence position
+    const GateToken gt = gate_token<T>(gr, 1, N, log_dt_scale[g.h], pos, kc);
+    WideRow<typename T::raw, 2 * NH> A;
+    WideRow<typename T::raw, NH> vp;
+#pragma unroll
+    for (int j = 0; j < NH; ++j) {
+      const Transition tr = gate_pair<T>(gr, 1, N, j, pos, gt, kc);
+      T::store(&A.e[2 * j], tr.ar);
+      T::store(&A.e[2 * j + 1], tr.ai);
+      T::store(&vp.e[j], tr.vp);
+    }
+    A.store(A_out + o * N);
+    vp.store(vp_out + o * NH);
+    T::store(beta_out + o, gt.beta);
+    T::store(selc_out + o, gt.selc);
+  } else {
+    const float pos = float(g.l + l0 + (l0_dev ? *l0_dev : 0)) * rope[g.h];
+    const GateToken gt = gate_token<T>(row, H, N, log_dt_scale[g.h], pos, kc);
+    for (int j = 0; j < Nh; ++j) {
+      const Transition tr = gate_pair<T>(row, H, N, j, pos, gt, kc);
+      T::store(A_out + o * N + 2 * j, tr.ar);
+      T::store(A_out + o * N + 2 * j + 1, tr.ai);
+      T::store(vp_out + o * Nh + j, tr.vp);
+    }
+    T::store(beta_out + o, gt.beta);
+    T::store(selc_out + o, gt.selc);
   }
-  T::store(beta_out + o, gt.beta);
-  T::store(selc_out + o, gt.selc);
 }
 
-template <typename T>
+// NH as in the forward: the gates, and the token's gradient rows whole, are requested before any is used.
+// B 8, L 2048, H 16, N 16, bf16 on MI355X: 29.4 -> 24.7 us.
+template <typename T, int NH>
 __global__ __launch_bounds__(256) void dynamics_bwd_kernel(
     const typename T::raw* __restrict__ gA, const typename T::raw* __restrict__ gvp,
     const typename T::raw* __restrict__ gbeta, const typename T::raw* __restrict__ gselc,
     const typename T::raw* __restrict__ gate, const float* __restrict__ log_dt_scale,
     const float* __restrict__ rope, typename T::raw* __restrict__ ggate, float* __restrict__ glog_terms,
-    float c, float omega_thresh, float adt_delta, float adt_smooth, float adt_eps, int L, int H, int N,
+    float c, float omega_thresh, float adt_delta, float adt_smooth, float adt_eps, int L, int H, int Nrt,
     int64_t total) {
   GateIdx g;
   if (!gate_idx(int64_t(blockIdx.x) * blockDim.x + threadIdx.x, L, H, total, g)) return;
+  const int N = NH > 0 ? 2 * NH : Nrt;
   const int Nh = N / 2, G = N + 5;
   const int64_t roff = g.bl * int64_t(G) * H + g.h;
   const typename T::raw* row = gate + roff;
-  typename T::raw* grow = ggate + roff;
   const int64_t o = g.bl * H + g.h;
+  // gate segment s, and the gradients of the token's A_bar and vp rows
+  constexpr int kHeld = NH > 0 ? NH : 1;
+  typename T::raw gr[2 * kHeld + 5];
+  WideRow<typename T::raw, 2 * kHeld> gAr;
+  WideRow<typename T::raw, kHeld> gvr;
+  if constexpr (NH > 0) {
+#pragma unroll
+    for (int s = 0; s < 2 * NH + 5; ++s) gr[s] = row[int64_t(s) * H];
+    gAr.load(gA + o * N);
+    gvr.load(gvp + o * NH);
+  }
+  auto seg = [&](int s) -> float {
+    if constexpr (NH > 0)
+      return T::load(&gr[s]);
+    else
+      return T::load(row + int64_t(s) * H);
+  };
+  typename T::raw* grow = ggate + roff;
   const float freq = rope[g.h];
   const float pos = float(g.l) * freq;
   const float log_scale = log_dt_scale[g.h];
 
-  const float selB = T::load(row + int64_t(N) * H), selC = T::load(row + int64_t(N + 1) * H);
-  const float seldt = T::load(row + int64_t(N + 2) * H), braw = T::load(row + int64_t(N + 3) * H);
-  const float rraw = T::load(row + int64_t(N + 4) * H);
+  const float selB = seg(N), selC = seg(N + 1);
+  const float seldt = seg(N + 2), braw = seg(N + 3);
+  const float rraw = seg(N + 4);
   const float rg = sigmoid(rraw);
-  const float a0raw = T::load(row);
+  const float a0raw = seg(0);
   const float a0 = softplus(a0raw);
-  const float w0 = T::load(row + int64_t(Nh) * H) + pos;
+  const float w0 = seg(Nh) + pos;
   const float dts = softplus(log_scale);
   const float wabs = fabsf(w0);
   const float chr = a0 + wabs + adt_eps;
@@ -111,10 +193,11 @@ __global__ __launch_bounds__(256) void dynamics_bwd_kernel(
   const float cr = c * rg;
   const float expo = 0.5f * (cr - 1.0f);
   float g_dt = 0.0f, g_r = 0.0f, ga0 = 0.0f, gw0 = 0.0f;
+#pragma unroll kHeld
   for (int j = 0; j < Nh; ++j) {
-    const float araw = T::load(row + int64_t(j) * H);
+    const float araw = seg(j);
     const float alpha = softplus(araw);
-    const float omega = T::load(row + int64_t(Nh + j) * H) + pos;
+    const float omega = seg(Nh + j) + pos;
     const float tau = 0.5f * dt;
     const float ac = fmaxf(alpha, 0.0f);
     const float ta = tau * ac, tw = tau * omega;
@@ -130,8 +213,16 @@ __global__ __launch_bounds__(256) void dynamics_bwd_kernel(
     const float scale = __builtin_amdgcn_exp2f(expo * lE2);
     const float eff = __builtin_amdgcn_exp2f(cr * lE2);
     const float vp = sqrtf(fmaxf(1.0f - eff, 1e-6f));
-    float gar = T::load(gA + o * N + 2 * j), gai = T::load(gA + o * N + 2 * j + 1);
-    const float gv = T::load(gvp + o * Nh + j);
+    float gar, gai, gv;
+    if constexpr (NH > 0) {
+      gar = T::load(&gAr.e[2 * j]);
+      gai = T::load(&gAr.e[2 * j + 1]);
+      gv = T::load(&gvr.e[j]);
+    } else {
+      gar = T::load(gA + o * N + 2 * j);
+      gai = T::load(gA + o * N + 2 * j + 1);
+      gv = T::load(gvp + o * Nh + j);
+    }
     const bool active = vp > 1e-6f && vp < 1.0f;
     const float d_eff = active ? gv * (-0.5f / vp) : 0.0f;
     const bool unclamped = E > 1e-8f;
@@ -276,6 +367,22 @@ namespace {
 using namespace cdssm;
 using namespace cdssm::gates;
 
+// go(NH) with NH = N / 2 where the kernels have it as a constant (N 2, 4, 8 or 16, rows of N elements at A and
+// of N / 2 at vp aligned for their wide accesses), else 0.
+template <typename Go>
+void by_pairs(int dtype, int64_t N, const void* A, const void* vp, Go&& go) {
+  const int64_t eb = dtype == 1 ? 2 : 4;
+  const auto aligned = [](const void* p, int64_t bytes) {
+    return reinterpret_cast<uintptr_t>(p) % uintptr_t(bytes < 16 ? bytes : 16) == 0;
+  };
+  const bool ok = aligned(A, N * eb) && aligned(vp, N / 2 * eb);
+  if (ok && N == 2) return go(std::integral_constant<int, 1>{});
+  if (ok && N == 4) return go(std::integral_constant<int, 2>{});
+  if (ok && N == 8) return go(std::integral_constant<int, 4>{});
+  if (ok && N == 16) return go(std::integral_constant<int, 8>{});
+  go(std::integral_constant<int, 0>{});
+}
+
 int check_dtype(const char* op, int dtype) {
   if (dtype != 0 && dtype != 1) {
     cdssm_host::set_error("%s: dtype must be 0 (fp32) or 1 (bf16), got %d", op, dtype);
@@ -325,16 +432,19 @@ extern "C" int cdssm_dynamics_fused_fwd_at(int dtype, const void* gate_raw, cons
   }
   const int64_t total = B * L * H;
   const unsigned blocks = unsigned((total + 255) / 256);
-  if (dtype == 1)
-    hipLaunchKernelGGL(dynamics_fwd_kernel<BF16>, dim3(blocks), dim3(256), 0, stream, (const uint16_t*)gate_raw,
-                       log_dt_scale, rope_freqs, (uint16_t*)A_bar, (uint16_t*)vp_scale, (uint16_t*)beta,
-                       (uint16_t*)sel_c, gating_c, omega_thresh, adt_delta, adt_smoothness, adt_eps, int(L),
-                       int(H), int(N), total, l0, l0_dev);
-  else
-    hipLaunchKernelGGL(dynamics_fwd_kernel<F32>, dim3(blocks), dim3(256), 0, stream, (const float*)gate_raw,
-                       log_dt_scale, rope_freqs, (float*)A_bar, (float*)vp_scale, (float*)beta, (float*)sel_c,
-                       gating_c, omega_thresh, adt_delta, adt_smoothness, adt_eps, int(L), int(H), int(N),
-                       total, l0, l0_dev);
+  by_pairs(dtype, N, A_bar, vp_scale, [&](auto nh) {
+    constexpr int NH = decltype(nh)::value;
+    if (dtype == 1)
+      hipLaunchKernelGGL((dynamics_fwd_kernel<BF16, NH>), dim3(blocks), dim3(256), 0, stream,
+                         (const uint16_t*)gate_raw, log_dt_scale, rope_freqs, (uint16_t*)A_bar, (uint16_t*)vp_scale,
+                         (uint16_t*)beta, (uint16_t*)sel_c, gating_c, omega_thresh, adt_delta, adt_smoothness,
+                         adt_eps, int(L), int(H), int(N), total, l0, l0_dev);
+    else
+      hipLaunchKernelGGL((dynamics_fwd_kernel<F32, NH>), dim3(blocks), dim3(256), 0, stream, (const float*)gate_raw,
+                         log_dt_scale, rope_freqs, (float*)A_bar, (float*)vp_scale, (float*)beta, (float*)sel_c,
+                         gating_c, omega_thresh, adt_delta, adt_smoothness, adt_eps, int(L), int(H), int(N), total,
+                         l0, l0_dev);
+  });
   return cdssm_host::check_launch(op);
 }
 
@@ -375,18 +485,21 @@ extern "C" int cdssm_dynamics_fused_bwd(int dtype, const void* grad_A_bar, const
   }
   const int64_t total = B * L * H;
   const unsigned blocks = unsigned((total + 255) / 256);
-  if (dtype == 1)
-    hipLaunchKernelGGL(dynamics_bwd_kernel<BF16>, dim3(blocks), dim3(256), 0, stream,
-                       (const uint16_t*)grad_A_bar, (const uint16_t*)grad_vp_scale, (const uint16_t*)grad_beta,
-                       (const uint16_t*)grad_sel_c, (const uint16_t*)gate_raw, log_dt_scale, rope_freqs,
-                       (uint16_t*)grad_gate_raw, workspace, gating_c, omega_thresh, adt_delta, adt_smoothness,
-                       adt_eps, int(L), int(H), int(N), total);
-  else
-    hipLaunchKernelGGL(dynamics_bwd_kernel<F32>, dim3(blocks), dim3(256), 0, stream, (const float*)grad_A_bar,
-                       (const float*)grad_vp_scale, (const float*)grad_beta, (const float*)grad_sel_c,
-                       (const float*)gate_raw, log_dt_scale, rope_freqs, (float*)grad_gate_raw, workspace,
-                       gating_c, omega_thresh, adt_delta, adt_smoothness, adt_eps, int(L), int(H), int(N),
-                       total);
+  by_pairs(dtype, N, grad_A_bar, grad_vp_scale, [&](auto nh) {
+    constexpr int NH = decltype(nh)::value;
+    if (dtype == 1)
+      hipLaunchKernelGGL((dynamics_bwd_kernel<BF16, NH>), dim3(blocks), dim3(256), 0, stream,
+                         (const uint16_t*)grad_A_bar, (const uint16_t*)grad_vp_scale, (const uint16_t*)grad_beta,
+                         (const uint16_t*)grad_sel_c, (const uint16_t*)gate_raw, log_dt_scale, rope_freqs,
+                         (uint16_t*)grad_gate_raw, workspace, gating_c, omega_thresh, adt_delta, adt_smoothness,
+                         adt_eps, int(L), int(H), int(N), total);
+    else
+      hipLaunchKernelGGL((dynamics_bwd_kernel<F32, NH>), dim3(blocks), dim3(256), 0, stream,
+                         (const float*)grad_A_bar, (const float*)grad_vp_scale, (const float*)grad_beta,
+                         (const float*)grad_sel_c, (const float*)gate_raw, log_dt_scale, rope_freqs,
+                         (float*)grad_gate_raw, workspace, gating_c, omega_thresh, adt_delta, adt_smoothness,
+                         adt_eps, int(L), int(H), int(N), total);
+  });
   st = cdssm_host::check_launch(op);
   if (st) return st;
   float* part = workspace + B * L * H;

@@ -174,3 +174,52 @@ def test_vp_clamp_gradient_matches_oracle():
     assert e <= 1e-3 and el <= 1e-3
     # outside the clamp heads nothing flows (their vp cotangent is zero)
     assert float(gg.reshape(B, L, N + 5, H)[..., ~clamp].abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("N", [2, 4, 8, 16])
+def test_whole_rows_equal_element_stores(dtype, N):
+    """State sizes 2, 4, 8 and 16 with aligned A_bar and vp rows run with the gates held and whole rows stored (or
+    loaded, in the backward); rows one element off their alignment run pair by pair.  The same expressions; a
+    product may be contracted into another of its sums, so the roundings (u = 2^-24) differ.  With c r <= 7.7:
+    mu is within 2 u, its factor E^((c r - 1) / 2) and the VP term E^(c r) within (4 c r + 16) u < 3e-6 of
+    themselves (4 u of E in the exponent, an exponent below 16 before they vanish), so A_bar and vp^2 agree to
+    3e-6, and after the rounding to bf16 to 2^-8 and 2^-7 of themselves more.  The gradients add terms of those,
+    each an error of 1e-5 of the largest at most (2^-8 after the rounding to bf16)."""
+    from cdssm_hip import _lib
+    lib, code = _lib.load(), _lib.DTYPE_CODE[dtype]
+    B, L, Hn = 2, 37, 5
+    gen = torch.Generator().manual_seed(N)
+    gate = torch.randn(B, L, (N + 5) * Hn, generator=gen).to(dtype).to(DEV)
+    lds, rope = torch.randn(Hn, generator=gen).to(DEV), torch.rand(Hn, generator=gen).to(DEV)
+    rows, consts = B * L * Hn, list(CONSTS.values())
+
+    def off(x, by):  # the same values, the base `by` elements past an aligned address
+        buf = torch.empty(x.numel() + 16, dtype=x.dtype, device=DEV)
+        out = buf[by:by + x.numel()]
+        out.copy_(x.reshape(-1))
+        return out
+
+    fwd, bwd = [], []
+    g = [torch.randn(rows * n, generator=gen).to(dtype).to(DEV) for n in (N, N // 2, 1, 1)]
+    ws = torch.empty(lib.cdssm_dynamics_fused_bwd_workspace_bytes(B, L, Hn) // 4, device=DEV)
+    for by in (0, 1):
+        outs = [off(torch.zeros(rows * n, dtype=dtype, device=DEV), by) for n in (N, N // 2, 1, 1)]
+        _lib.check(lib.cdssm_dynamics_fused_fwd(code, _lib.ptr(gate), _lib.ptr(lds), _lib.ptr(rope), *consts,
+                                                *[_lib.ptr(x) for x in outs], B, L, Hn, N,
+                                                _lib.stream_of(gate.device)), "fwd")
+        gi = [off(x, by) for x in g]
+        gg, gl = torch.zeros_like(gate), torch.zeros(Hn, device=DEV)
+        _lib.check(lib.cdssm_dynamics_fused_bwd(code, *[_lib.ptr(x) for x in gi], _lib.ptr(gate), _lib.ptr(lds),
+                                                _lib.ptr(rope), *consts, _lib.ptr(gg), _lib.ptr(gl), _lib.ptr(ws),
+                                                B, L, Hn, N, _lib.stream_of(gate.device)), "bwd")
+        torch.cuda.synchronize()
+        fwd.append(outs)
+        bwd.append((gg, gl))
+    ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 0.0
+    for i, (a, b) in enumerate(zip(*[[x.double() for x in f] for f in fwd])):
+        a, b, u = (a * a, b * b, 2 * ulp) if i == 1 else (a, b, ulp)
+        assert bool(((a - b).abs() <= 3e-6 + u * a.abs()).all()), f"output {i}"
+    scale = bwd[0][0].float().abs().max()  # the gradients' sums over pairs: rounding against the largest
+    assert (bwd[0][0].float() - bwd[1][0].float()).abs().max() <= (2.0 ** -8 if dtype == torch.bfloat16 else 1e-5) * scale
+    assert torch.allclose(bwd[0][1], bwd[1][1], rtol=1e-4, atol=1e-4 * float(bwd[0][1].abs().max()))
