@@ -249,3 +249,20 @@ def test_conv1d_silu_backward_vector_and_scalar_paths_agree_bitwise(dtype, K):
     torch.cuda.synchronize()
     for a, c in zip(ga, gb):
         assert torch.equal(a, c)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("L,K", [(1, 1), (1, 8), (2, 4), (7, 3), (8, 4), (9, 4), (17, 8), (24, 2)])
+def test_conv1d_silu_rows_and_weights_held(dtype, L, K):
+    """Token blocks of 8 with every row and weight requested ahead, at the edges of a block and of the sequence.
+    Weights off a 16-byte boundary are read one element at a time: the same sums in the same order, equal bits."""
+    from cdssm_hip.lm import conv1d_silu
+    B, C = 2, 48
+    g = torch.Generator().manual_seed(10 * L + K)
+    x, b = torch.randn(B, L, C, generator=g).to(dtype), torch.randn(C, generator=g).to(dtype)
+    w = torch.randn(C, K, generator=g).to(dtype)
+    held = torch.empty(C * K + 1, dtype=dtype, device=DEV)
+    held[1:] = w.reshape(-1).to(DEV)
+    y = conv1d_silu(x.to(DEV), w.to(DEV), b.to(DEV))
+    assert torch.equal(y, conv1d_silu(x.to(DEV), held[1:].view(C, K), b.to(DEV)))
+    assert rel(y.cpu(), lo.conv1d_silu(x.double(), w.double(), b.double())) < _tol(dtype)
