@@ -322,6 +322,32 @@ def skinny_linear(x: Tensor, weight: Tensor, bias: Optional[Tensor] = None, resi
     return y
 
 
+def skinny_linear_conv_step(x: Tensor, weight: Tensor, bias: Optional[Tensor], norm_weight: Tensor, eps: float,
+                            conv_col: int, window: Tensor, conv_weight: Tensor, conv_bias: Tensor) -> tuple:
+    """``skinny_linear`` with a norm weight, and ``conv1d_silu_step`` on its columns conv_col .. conv_col + C, in
+    one launch (cdssm_skinny_gemm_conv_step): (product (M, N), conv output (M, C)), window (M, K-1, C) updated in
+    place.  The same bits as the two calls."""
+    if not _skinny_ok(x, weight):
+        raise ValueError("skinny_linear_conv_step: needs bf16 x (M <= 64, K % 128 == 0) and weight with aligned rows")
+    M, K = x.shape
+    N = weight.shape[0]
+    taps, C = conv_weight.shape[-1], conv_bias.shape[0]
+    if tuple(window.shape) != (M, taps - 1, C) or window.dtype != x.dtype or not window.is_contiguous():
+        raise ValueError(f"window must be a contiguous ({M}, {taps - 1}, {C}) {x.dtype} tensor")
+    b = None if bias is None else bias.to(torch.bfloat16).contiguous()
+    g = norm_weight.to(torch.bfloat16).contiguous()
+    wc = conv_weight.to(torch.bfloat16).contiguous()
+    bc = conv_bias.to(torch.bfloat16).contiguous()
+    y = torch.empty(M, N, dtype=torch.bfloat16, device=x.device)
+    yc = torch.empty(M, C, dtype=torch.bfloat16, device=x.device)
+    st = _lib.load().cdssm_skinny_gemm_conv_step(1, _lib.ptr(x), x.stride(0), _lib.ptr(weight), weight.stride(0),
+                                                 _lib.ptr(b), _lib.ptr(g), float(eps), _lib.ptr(y), N, M, N, K,
+                                                 conv_col, _lib.ptr(window), _lib.ptr(wc), _lib.ptr(bc), _lib.ptr(yc),
+                                                 C, taps, _lib.stream_of(x.device))
+    _lib.check(st, "cdssm_skinny_gemm_conv_step")
+    return y, yc
+
+
 def _wgrad_slabs(T: int, O: int, I: int) -> int:
     """Token slabs of a weight gradient dW = dY^T X over T tokens (O x I output).  One GEMM with an O x I
     output of at most 1024 x 1024 and T = 16384 leaves most CUs idle (hipBLASLt: 64 x 64 tiles, no split
@@ -1185,15 +1211,18 @@ class CDSSMBlock(nn.Module):
         cfg = self.config
         N, H, D, Di = cfg.state_dim, cfg.n_heads, cfg.head_dim, cfg.d_inner
         B = x.shape[0]
-        if _skinny_ok(x, self.in_proj.weight):  # RMSNorm + in_proj in one skinny product
-            proj = skinny_linear(x, self.in_proj.weight, self.in_proj.bias, norm_weight=self.norm.weight,
-                                 eps=self.norm.eps)
+        x_conv = None
+        if _skinny_ok(x, self.in_proj.weight):  # RMSNorm + in_proj + the conv's step in one skinny product
+            proj, x_conv = skinny_linear_conv_step(x, self.in_proj.weight, self.in_proj.bias, self.norm.weight,
+                                                   self.norm.eps, Di, cache["conv"], self.conv.weight,
+                                                   self.conv.bias)
         else:
             proj = self.in_proj(rms_norm(x, self.norm.weight, self.norm.eps))  # (B, 3 Di + H N)
         z, x_gate, K, V = proj.split([Di, Di, Di, H * N], dim=-1)
         K = K.reshape(B, 1, H, D)
         V = V.reshape(B, H, N)
-        x_conv = conv1d_silu_step(x_gate, cache["conv"], self.conv.weight, self.conv.bias)
+        if x_conv is None:
+            x_conv = conv1d_silu_step(x_gate, cache["conv"], self.conv.weight, self.conv.bias)
         GH = (N + 5) * H
         if _skinny_ok(x_conv, cache["w_gq"]):
             gq = skinny_linear(x_conv, cache["w_gq"], cache["b_gq"])  # (B, GH + Di): gates | Q

@@ -760,6 +760,18 @@ int cdssm_skinny_gemm(int dtype, const void* X, int64_t ldx, const void* W, int6
                       int64_t N, int64_t K, hipStream_t stream);
 
 /*
+ * cdssm_skinny_gemm (no R) and, in the same launch, cdssm_conv1d_silu_step on
+ * the rounded columns conv_col .. conv_col + C - 1 of Y: window (M, taps - 1,
+ * C), conv_weight (C, taps), conv_bias (C), conv_y (M, C), all bf16 and dense,
+ * 1 <= taps <= 8.  The same bits as the two calls.  The decode step's in_proj
+ * with the conv of its x_gate columns (block.py:155-160).
+ */
+int cdssm_skinny_gemm_conv_step(int dtype, const void* X, int64_t ldx, const void* W, int64_t ldw, const void* bias,
+                                const void* wnorm, float eps, void* Y, int64_t ldy, int64_t M, int64_t N, int64_t K,
+                                int64_t conv_col, void* window, const void* conv_weight, const void* conv_bias,
+                                void* conv_y, int64_t C, int64_t taps, hipStream_t stream);
+
+/*
  * One decode token of the model block's scan path in one launch, per (b, h):
  * the gate-level dynamics at the device-held position (as
  * cdssm_dynamics_fused_fwd_at), K/Q normalisation and q.k (as

@@ -116,3 +116,26 @@ def test_rows_per_workgroup_leave_the_sums_alone(M, N, norm):
         x64 = x64 * torch.rsqrt(x64.pow(2).mean(-1, keepdim=True) + 1e-5) * nw.double()
     ref = (x64 @ w.double().t() + bias.double() + res.double()).cpu()
     assert rel(y.double().cpu(), ref) <= (2 if norm else 1) * 2.0 ** -8 + 1e-5
+
+
+@pytest.mark.parametrize("M,N,col,C,taps", [
+    (64, 3104, 1024, 1024, 4),  # in_proj of the decode step; 64 rows per workgroup
+    (33, 45, 7, 30, 8), (1, 16, 0, 16, 1), (17, 40, 24, 16, 2), (64, 2304, 1, 2303, 3),
+])
+def test_conv_step_in_the_product(M, N, col, C, taps):
+    """The product and the conv step on its columns in one launch, over two tokens, against the two launches: the
+    same arithmetic on the same rounded values, equal bits in the product, the conv's output and the window."""
+    from cdssm_hip.lm import conv1d_silu_step, skinny_linear, skinny_linear_conv_step
+    K, g = 256, torch.Generator().manual_seed(N + taps)
+
+    def rnd(*s):
+        return torch.randn(*s, generator=g).to(torch.bfloat16).to(DEV)
+
+    w, b, nw, cw, cb, win = rnd(N, K), rnd(N), rnd(K), rnd(C, 1, taps), rnd(C), rnd(M, taps - 1, C)
+    win2 = win.clone()
+    for _ in range(2):
+        x = rnd(M, K)
+        y, yc = skinny_linear_conv_step(x, w, b, nw, 1e-5, col, win, cw, cb)
+        want = skinny_linear(x, w, b, norm_weight=nw, eps=1e-5)
+        assert torch.equal(y, want)
+        assert torch.equal(yc, conv1d_silu_step(want[:, col:col + C], win2, cw, cb)) and torch.equal(win, win2)
