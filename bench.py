@@ -37,6 +37,7 @@ for _p in (ROOT, PKG_DIR):
 
 HBM_PEAK_GBS = 8000.0  # MI355X HBM3E, vendor peak
 TRAFFIC_FILES = {
+    "mf_onepass_kernel": os.path.join(ROOT, "profiles", "mfma_forward_C1_counters.md"),
     "fused_fwd_onepass_kernel": os.path.join(ROOT, "profiles", "fused_fwd_onepass_C1_hbm_traffic.txt"),
     "fused_fwd_main_kernel": os.path.join(ROOT, "profiles", "fused_fwd_main_C1_hbm_traffic.txt"),
 }
@@ -55,7 +56,10 @@ def recorded_traffic(path, key="traffic_bytes_per_launch"):
 
 
 FWD_BWD_TRAFFIC = os.path.join(ROOT, "profiles", "fused_fwd_bwd_C1_C2_hbm_traffic.txt")
-MFMA_PROFILE = os.path.join(ROOT, "profiles", "fused_fwd_onepass_C1_sq_counters.md")
+MFMA_PROFILES = {
+    "mf_onepass_kernel": os.path.join(ROOT, "profiles", "mfma_forward_C1_counters.md"),
+    "fused_fwd_onepass_kernel": os.path.join(ROOT, "profiles", "fused_fwd_onepass_C1_sq_counters.md"),
+}
 MFMA_VARIANT_PROFILE = os.path.join(ROOT, "profiles", "mfma_correction_vs_sequential_C1_C2.md")
 CHUNKED_PROFILE = os.path.join(ROOT, "profiles", "chunked_scan_n16_C4_counters.md")
 
@@ -64,11 +68,11 @@ def mfma_util(kernel):
     """MFMA utilisation of the forward kernel the bench times, from committed SQ counters (rocprofv3 cannot
     run inside this process): MFMA FLOPs / kernel time / 2.5 PFLOP/s dense bf16, with the path named.  The
     chunked MFMA correction (not the default) is quoted beside it."""
-    return {"path": kernel + " (sequential correction: no MFMA instructions)"
-            if kernel == "fused_fwd_onepass_kernel" else kernel,
-            "value": recorded_traffic(MFMA_PROFILE, "mfma_util"),
-            "mfma_insts_per_wave": recorded_traffic(MFMA_PROFILE, "mfma_insts_per_wave"),
-            "source": os.path.relpath(MFMA_PROFILE, ROOT),
+    source = MFMA_PROFILES.get(kernel)
+    return {"path": kernel + (" (sequential: no MFMA instructions)" if kernel == "fused_fwd_onepass_kernel" else ""),
+            "value": source and recorded_traffic(source, "mfma_util"),
+            "mfma_insts_per_wave": source and recorded_traffic(source, "mfma_insts_per_wave"),
+            "source": source and os.path.relpath(source, ROOT),
             "chunked_mfma_correction": {"path": "four_launch_mfma (fused_fwd_corr_sweep_kernel, not default)",
                                         "value": recorded_traffic(MFMA_VARIANT_PROFILE, "mfma_util_C1"),
                                         "source": os.path.relpath(MFMA_VARIANT_PROFILE, ROOT)},
@@ -888,7 +892,12 @@ def main():
     phases = run.profile(args.steps)
     main_ms = phases["main"]
     one_pass = all(phases[k] == 0.0 for k in ("summary", "carry_fold", "carry_replay"))
-    kernel = "fused_fwd_onepass_kernel" if one_pass else "fused_fwd_main_kernel"
+    # one launch: on the matrix cores where one round of workgroups (two per CU at D = 64, one at 128) takes
+    # every segment of 4 chunks and 4 heads, else the sequential kernel
+    n_cu = torch.cuda.get_device_properties(dev).multi_processor_count
+    items = cfg.B * -(-cfg.L // (4 * cfg.D)) * -(-cfg.H // 4)
+    matrix = args.forward_path == "auto" and items <= n_cu * (2 if cfg.D == 64 else 1)
+    kernel = ("mf_onepass_kernel" if matrix else "fused_fwd_onepass_kernel") if one_pass else "fused_fwd_main_kernel"
     traffic_file = TRAFFIC_FILES[kernel]
 
     tokens = cfg.B * cfg.L

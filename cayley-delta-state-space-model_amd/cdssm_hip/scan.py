@@ -273,11 +273,12 @@ _path_generation = [0]
 def set_forward_path(path: str) -> str:
     """Select how the inference forward is launched; returns the previous setting.
 
-    "auto" (default) takes the one-pass forward where one round of resident
-    workgroups holds every segment of 4 chunks (and, for inference, where the
-    persistent one-pass fills whole rounds), else the four-launch scan;
-    "four_launch" always takes the multi-launch passes; "one_pass" requires
-    the one-launch passes (calls they cannot serve raise); "four_launch_mfma"
+    "auto" (default) takes a one-launch forward where one round of resident
+    workgroups holds every segment of 4 chunks (for scan-level bf16 inference
+    the matrix-core form, whose y differs from the sequential forms' by the
+    order of its sums; else the sequential one-pass, for inference also where
+    it fills whole persistent rounds), else the four-launch scan; "four_launch" always takes the multi-launch passes; "one_pass" requires
+    the sequential one-launch passes (calls they cannot serve raise); "four_launch_mfma"
     takes the multi-launch passes with the correction as the chunked MFMA
     pass (bf16 inference forward, chunk a multiple of 16 up to 128; other calls
     raise).  Process-wide; the same choice applies to the backward's correction
@@ -331,7 +332,7 @@ class PreparedForward:
     validation, allocation or tensor creation on the host: the launch path for
     serving loops, graph capture and timing.  The bound tensors must stay alive
     and keep their shapes.  The first call draws the one-launch pass's look-back
-    epoch with a kernel of its own (cdssm_fused_scan_fwd); later calls reuse
+    epoch (cdssm_fused_scan_fwd); later calls reuse
     the epoch the previous call left in the workspace it owns
     (cdssm_fused_scan_fwd_continue): one launch per call.
     """

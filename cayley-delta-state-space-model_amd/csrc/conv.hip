@@ -66,9 +66,9 @@ __device__ __forceinline__ void store_vec(typename T::raw* p, const float (&x)[V
 }
 
 // Memory bounds it (x once and its halo, y once).  A thread requests all of its rows, then its weights, before
-// it uses any: with a row's load behind the previous row's arithmetic, and the weights in loads of one element,
-// a call came at 3.3 to 3.5 of the 5.1 TB/s that a copy reaches.  B 8, L 2048, C 1024, K 4, bf16 on MI355X:
-// 19.1 -> 18.1 us; B 4, L 2048, C 1536: 15.6 -> 13.9 us.
+// it uses any; with a row's load behind the previous row's arithmetic, and the weights in loads of one element,
+// a call came at 3.3 to 3.5 of the 5.1 TB/s that a copy reaches.  K 4, bf16 on MI355X: B 8, L 2048, C 1024
+// 18.9 -> 18.1 us, B 4, L 2048, C 1536 15.3 -> 13.9.
 template <typename T, int VEC, int K>
 __global__ __launch_bounds__(256) void conv1d_silu_fwd_kernel(const typename T::raw* __restrict__ x,
                                                               const typename T::raw* __restrict__ w,

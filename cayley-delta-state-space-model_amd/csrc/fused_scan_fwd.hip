@@ -948,10 +948,11 @@ __global__ __launch_bounds__(kWave) void fused_fwd_corr_sweep_kernel(
 // entering every chunk and G_k (the four-launch layout), the per-token records
 // (p_t, pc_t), (c^_{t+1}.q_t, Y_t.q_t) and g_t, as the main pass does.
 // Flags hold epoch << 3 | bits (kFlagMap, kFlagLeave, kFlagGroup) with a
-// per-call epoch read from the look-back area's control block, where
-// fwd_epoch_kernel (launched just before, on the same stream) writes it from a
-// device-side counter; so the workspace needs no clearing between calls and a
-// captured HIP graph draws a new epoch on every replay.  Published
+// per-call epoch: an argument of the launch (eager calls, draw_call_epoch) or
+// read from the look-back area's control block, where fwd_epoch_kernel
+// (launched just before, on the same stream) writes it from a device-side
+// counter; so the workspace needs no clearing between calls and a captured HIP
+// graph draws a new epoch on every replay.  Published
 // data and flags are written and read with agent-scope atomics (stores written
 // through to the device-coherent level, loads served from it), so no cache
 // maintenance is needed: a writer waits until its data stores are acknowledged
@@ -1691,8 +1692,7 @@ int launch_fused_fwd(const void* q, const void* k, const void* v, const void* be
 // on a GPU uses that GPU's copy, so such calls must not overlap on one GPU.
 // Nothing in it needs clearing between calls: the carry arrays are written
 // before they are read in each call, and the look-back flags only count when
-// they carry the running call's epoch (fresh per call, written by the epoch
-// kernel into the area's control block).
+// they carry the running call's epoch (fresh per call).
 // ---------------------------------------------------------------------------
 constexpr size_t kScratchBytes = size_t(32) << 20;  // 32 MiB
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];

@@ -175,10 +175,11 @@ int cdssm_fused_scan_fwd_train(int dtype, const void* q, const void* k, const vo
  * untouched since.  No counterpart in the reference: for callers that keep a
  * workspace across calls (serving loops, training steps, captured graphs).
  * Every one-launch pass draws a look-back epoch, a tag that tells this call's
- * flags from earlier calls' in the never-cleared workspace; the entries above
- * launch a one-thread kernel for it, while these reuse the one that the
- * previous call's last workgroup left in the workspace (one launch per call
- * instead of two).  Results are bit-identical to the entries above.  Calling
+ * flags from earlier calls' in the never-cleared workspace.  The entries above
+ * draw it on the host and pass it to the kernel or, where the stream is being
+ * captured, launch a one-thread kernel for it; these reuse the one that the
+ * previous call's last workgroup left in the workspace (one launch under
+ * capture instead of two).  Results are bit-identical to the entries above.  Calling
  * them on a workspace that has not held such a call, or whose contents were
  * changed since, may read stale look-back flags as ready.
  */
@@ -317,7 +318,7 @@ int cdssm_fused_scan_bwd_profile(int dtype, const void* q, const void* k, const 
 
 /*
  * Instrumentation (no counterpart in the reference): cdssm_fused_scan_fwd
- * (with its epoch kernel), recording for every wave of the one-pass kernel the
+ * recording for every wave of the one-launch kernel the
  * 100 MHz real-time counter (s_memrealtime) at 8 points of its segment: entry,
  * staging done, local pass done, segment map published, look-back wait done,
  * carry folded, correction pass done, segment end.  stamps: device memory of
@@ -366,10 +367,12 @@ int cdssm_fused_scan_fwd_set_path(int mode);
  * with the device (device-to-host copies), so it must not be called while the
  * stream is being captured into a graph.
  *
- * The one-launch passes draw their flag epoch on the device: a one-thread
- * kernel launched on the same stream just before the pass writes a fresh
- * epoch from a per-device counter into the workspace, so the workspace needs
- * no clearing between calls and a captured graph stays correct on every replay.
+ * The one-launch passes tag their flags with an epoch of the call, so the
+ * workspace needs no clearing between calls.  An eager call takes it from a
+ * counter of the process and passes it by value; a captured call launches a
+ * one-thread kernel just before the pass that writes one from a per-device
+ * counter into the workspace, so a graph draws a new one on every replay.  The
+ * two kinds differ in one bit and never meet.
  */
 int cdssm_lookback_status(int clear, int* status);
 
