@@ -1200,10 +1200,10 @@ __device__ __forceinline__ void onepass_segment(const OnePassArgs<T>& a, int ite
       const float4 g = GF[u * HPW + hh];
 #pragma unroll
       for (int j = 0; j < DPL; ++j) {
-        const float2 f = Fx[u * SEGN + hh * D + sub * DPL + j];
-        const float nr = g.x * cr[j] - g.y * ci[j] + f.x;
-        ci[j] = g.x * ci[j] + g.y * cr[j] + f.y;
-        cr[j] = nr;
+        const float2 n = map_apply<false>(make_float2(g.x, g.y), make_float2(cr[j], ci[j]),
+                                          Fx[u * SEGN + hh * D + sub * DPL + j]);
+        cr[j] = n.x;
+        ci[j] = n.y;
       }
     }
     if (!hok) {

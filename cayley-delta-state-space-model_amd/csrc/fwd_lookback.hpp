@@ -34,6 +34,23 @@ __device__ __forceinline__ bool watch_flags(const unsigned long long* f0, int H,
   }
 }
 
+// G s + F, the state s after the map (G, F).  Its roundings are spelled out: where the compiler forms the
+// multiply-adds, which of two products keeps its own rounding changes with the code around them, and with it
+// the bits of every later output (24 bf16 layers make 1e-2 of one such change).  IM_RE: the imaginary part's
+// fma takes the state's real part, else its imaginary part.
+template <bool IM_RE>
+__device__ __forceinline__ float2 map_apply(float2 G, float2 s, float2 F) {
+#pragma clang fp contract(off)
+  const float re = fmaf(G.x, s.x, -(G.y * s.y));
+  const float im = IM_RE ? fmaf(G.y, s.x, G.x * s.y) : fmaf(G.x, s.y, G.y * s.x);
+  return make_float2(re + F.x, im + F.y);
+}
+// G H, the product of two maps' rotations.
+__device__ __forceinline__ float2 map_product(float2 G, float2 H) {
+#pragma clang fp contract(off)
+  return make_float2(fmaf(G.x, H.x, -(G.y * H.y)), fmaf(G.x, H.y, G.y * H.x));
+}
+
 // Phase stamps of cdssm_fused_scan_fwd_stamped: segment entry, staging done,
 // local pass done, segment map published, look-back wait done, carry folded,
 // correction pass done, segment end.
@@ -56,6 +73,7 @@ __device__ __forceinline__ void segment_carry(const OnePassBufs& ob, const float
   constexpr int SEGN = HPW * D;                  // complex elements of a head group's state
   constexpr int EPT = SEGN / (kWave * kOnePassW);  // of which each thread composes EPT
   static_assert(EPT >= 1 && EPT * kWave * kOnePassW == SEGN, "segment state tiles the workgroup");
+  constexpr bool RE = EPT > 1;                   // map_apply's order in the folds across segments
   const int lane = int(threadIdx.x) % kWave;
   // 2. segment map over the live chunks; thread x composes elements
   // e = x * EPT + i of the head group's state (head e / D, element e % D)
@@ -72,11 +90,8 @@ __device__ __forceinline__ void segment_carry(const OnePassBufs& ob, const float
     const float4 g = GF[u * HPW + ej];
     const float2 gu = make_float2(g.x, g.y);
 #pragma unroll
-    for (int i = 0; i < EPT; ++i) {
-      const float2 f = Fx[u * SEGN + e0 + i];
-      segF[i] = make_float2(gu.x * segF[i].x - gu.y * segF[i].y + f.x, gu.x * segF[i].y + gu.y * segF[i].x + f.y);
-    }
-    segG = make_float2(gu.x * segG.x - gu.y * segG.y, gu.x * segG.y + gu.y * segG.x);
+    for (int i = 0; i < EPT; ++i) segF[i] = map_apply<false>(gu, segF[i], Fx[u * SEGN + e0 + i]);
+    segG = map_product(gu, segG);
   }
   const int64_t sb0 = (int64_t(bi) * NSEG + seg) * H;  // (b, seg, head 0)
   unsigned long long* flag = ob.flag + sb0 + hbase;
@@ -137,11 +152,8 @@ __device__ __forceinline__ void segment_carry(const OnePassBufs& ob, const float
       for (int u = 0; u < kFwdGroup; ++u) {
         const float2 gu = u < kFwdGroup - 1 ? G[u] : segG;
 #pragma unroll
-        for (int i = 0; i < EPT; ++i) {
-          const float2 f = u < kFwdGroup - 1 ? F[u][i] : segF[i];
-          Fg[i] = make_float2(gu.x * Fg[i].x - gu.y * Fg[i].y + f.x, gu.x * Fg[i].y + gu.y * Fg[i].x + f.y);
-        }
-        Gg = make_float2(gu.x * Gg.x - gu.y * Gg.y, gu.x * Gg.y + gu.y * Gg.x);
+        for (int i = 0; i < EPT; ++i) Fg[i] = map_apply<RE>(gu, Fg[i], u < kFwdGroup - 1 ? F[u][i] : segF[i]);
+        Gg = map_product(gu, Gg);
       }
       if (!okg) {
 #pragma unroll
@@ -237,8 +249,7 @@ __device__ __forceinline__ void segment_carry(const OnePassBufs& ob, const float
       if (u < ngrp + nmap) {
 #pragma unroll
         for (int i = 0; i < EPT; ++i)
-          Sin[i] = make_float2(G[u].x * Sin[i].x - G[u].y * Sin[i].y + F[u][i].x,
-                               G[u].x * Sin[i].y + G[u].y * Sin[i].x + F[u][i].y);
+          Sin[i] = u == 0 ? map_apply<false>(G[u], Sin[i], F[u][i]) : map_apply<RE>(G[u], Sin[i], F[u][i]);
       }
     }
     if (!ok) {
@@ -254,8 +265,7 @@ __device__ __forceinline__ void segment_carry(const OnePassBufs& ob, const float
   if (ehok && (anchor_end || seg + 1 == NSEG)) {
 #pragma unroll
     for (int i = 0; i < EPT; ++i) {
-      const float2 so = make_float2(segG.x * Sin[i].x - segG.y * Sin[i].y + segF[i].x,
-                                    segG.x * Sin[i].y + segG.y * Sin[i].x + segF[i].y);
+      const float2 so = map_apply<RE>(segG, Sin[i], segF[i]);
       if (anchor_end) {
         st_agent(ob.seg_s + (sb0 + eh) * D + ed + i, so);
       } else {

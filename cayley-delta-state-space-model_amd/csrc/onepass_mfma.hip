@@ -774,8 +774,9 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
       for (int u = 0; u < wv; ++u) {
         const float4 G = GF[u * kMfHeads + g];
         const float4 F = *reinterpret_cast<const float4*>(&Fx[u * SEGN + e0]);
-        s = make_float4(G.x * s.x - G.y * s.y + F.x, G.x * s.y + G.y * s.x + F.y, G.x * s.z - G.y * s.w + F.z,
-                        G.x * s.w + G.y * s.z + F.w);
+        const float2 n0 = map_apply<false>(make_float2(G.x, G.y), make_float2(s.x, s.y), make_float2(F.x, F.y));
+        const float2 n1 = map_apply<false>(make_float2(G.x, G.y), make_float2(s.z, s.w), make_float2(F.z, F.w));
+        s = make_float4(n0.x, n0.y, n1.x, n1.y);
       }
       if (!hok) s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
       st[ks][0] = f32x4_t{0.0f, 0.0f, s.x, s.y};
