@@ -266,9 +266,8 @@ __device__ __forceinline__ void decode_token_wave(
   }
 
   // dynamics at the token's position, rounded as DynamicsFusedFn stores them
-  const float pp = float(l) * rope;
-  const gates::GateToken gt = gates::gate_token<T>(gr, 1, N, lds, pp, a.kc);
-  const Transition tr0 = gates::gate_pair<T>(gr, 1, N, 0, pp, gt, a.kc);
+  const gates::GateToken gt = gates::gate_token<T>(gr, 1, N, lds, float(l), rope, a.kc);
+  const Transition tr0 = gates::gate_pair<T>(gr, 1, N, 0, gates::rope_angle(float(l), rope), gt, a.kc);
   const Transition tr{round_to<T>(tr0.ar), round_to<T>(tr0.ai), round_to<T>(tr0.vp)};
   const float bb = round_to<T>(gt.beta), sc = round_to<T>(gt.selc);
 

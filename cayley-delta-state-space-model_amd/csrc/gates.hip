@@ -98,8 +98,8 @@ __global__ __launch_bounds__(256) void dynamics_fwd_kernel(
     typename T::raw gr[2 * NH + 5];
 #pragma unroll
     for (int s = 0; s < 2 * NH + 5; ++s) gr[s] = row[int64_t(s) * H];
-    const float pos = float(g.l + l0 + (l0_dev ? *l0_dev : 0)) * rope[g.h];  // sequence position
-    const GateToken gt = gate_token<T>(gr, 1, N, log_dt_scale[g.h], pos, kc);
+    const float l = float(g.l + l0 + (l0_dev ? *l0_dev : 0)), freq = rope[g.h], pos = rope_angle(l, freq);
+    const GateToken gt = gate_token<T>(gr, 1, N, log_dt_scale[g.h], l, freq, kc);
     WideRow<typename T::raw, 2 * NH> A;
     WideRow<typename T::raw, NH> vp;
 #pragma unroll
@@ -114,8 +114,8 @@ __global__ __launch_bounds__(256) void dynamics_fwd_kernel(
     T::store(beta_out + o, gt.beta);
     T::store(selc_out + o, gt.selc);
   } else {
-    const float pos = float(g.l + l0 + (l0_dev ? *l0_dev : 0)) * rope[g.h];
-    const GateToken gt = gate_token<T>(row, H, N, log_dt_scale[g.h], pos, kc);
+    const float l = float(g.l + l0 + (l0_dev ? *l0_dev : 0)), freq = rope[g.h], pos = rope_angle(l, freq);
+    const GateToken gt = gate_token<T>(row, H, N, log_dt_scale[g.h], l, freq, kc);
     for (int j = 0; j < Nh; ++j) {
       const Transition tr = gate_pair<T>(row, H, N, j, pos, gt, kc);
       T::store(A_out + o * N + 2 * j, tr.ar);
@@ -163,7 +163,7 @@ __global__ __launch_bounds__(256) void dynamics_bwd_kernel(
   };
   typename T::raw* grow = ggate + roff;
   const float freq = rope[g.h];
-  const float pos = float(g.l) * freq;
+  const float pos = rope_angle(float(g.l), freq);
   const float log_scale = log_dt_scale[g.h];
 
   const float selB = seg(N), selC = seg(N + 1);
@@ -172,7 +172,7 @@ __global__ __launch_bounds__(256) void dynamics_bwd_kernel(
   const float rg = sigmoid(rraw);
   const float a0raw = seg(0);
   const float a0 = softplus(a0raw);
-  const float w0 = seg(Nh) + pos;
+  const float w0 = fmaf(float(g.l), freq, seg(Nh));
   const float dts = softplus(log_scale);
   const float wabs = fabsf(w0);
   const float chr = a0 + wabs + adt_eps;
@@ -193,8 +193,7 @@ __global__ __launch_bounds__(256) void dynamics_bwd_kernel(
   const float cr = c * rg;
   const float expo = 0.5f * (cr - 1.0f);
   float g_dt = 0.0f, g_r = 0.0f, ga0 = 0.0f, gw0 = 0.0f;
-#pragma unroll kHeld
-  for (int j = 0; j < Nh; ++j) {
+  auto pair = [&](int j) {
     const float araw = seg(j);
     const float alpha = softplus(araw);
     const float omega = seg(Nh + j) + pos;
@@ -255,7 +254,14 @@ __global__ __launch_bounds__(256) void dynamics_bwd_kernel(
       T::store(grow + int64_t(j) * H, ga_raw);
       T::store(grow + int64_t(Nh + j) * H, gw_raw);
     }
+  };
+  if constexpr (NH > 0) {
+#pragma unroll
+    for (int j = 0; j < NH; ++j) pair(j);
+  } else {
+    for (int j = 0; j < Nh; ++j) pair(j);
   }
+  asm("" : "+v"(ga0), "+v"(gw0));  // values by now: not to be joined with the sums below
   // adaptive dt
   const float g_seldt = g_dt * sigmoid(seldt);
   const float capf = capped ? 1.0f : 0.0f;
