@@ -562,6 +562,13 @@ __device__ __forceinline__ Transition cayley_gated(float dt, float r, float alph
   return o;
 }
 
+// g a, complex, with its roundings spelled out: where the compiler forms the multiply-adds, which of the
+// imaginary part's products keeps its own rounding changes with the code around them.
+__device__ __forceinline__ float2 rotate(float2 g, float2 a) {
+#pragma clang fp contract(off)
+  return make_float2(fmaf(g.x, a.x, -(g.y * a.y)), fmaf(g.x, a.y, g.y * a.x));
+}
+
 // ---------------------------------------------------------------------------
 // Segment look-back between the workgroups of a one-launch pass.
 // ---------------------------------------------------------------------------

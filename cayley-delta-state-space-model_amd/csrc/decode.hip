@@ -121,7 +121,7 @@ __global__ __launch_bounds__(kWave) void decode_step_kernel(
   zqi = group_sum<LPH>(zqi);
   const float yr = sc * (zqr + (g.x * cqr - g.y * cqi));
   const float yi = sc * (zqi + (g.x * cqi + g.y * cqr));
-  const float2 gn = make_float2(g.x * tr.ar - g.y * tr.ai, g.x * tr.ai + g.y * tr.ar);
+  const float2 gn = rotate(g, make_float2(tr.ar, tr.ai));
 
   if (!hok) return;  // nothing below reduces across lanes
   if (sub == 0) {
@@ -336,7 +336,7 @@ __device__ __forceinline__ void decode_token_wave(
   zqi = group_sum<LPH>(zqi);
   const float yr = round_to<T>(sc * (zqr + (g.x * cqr - g.y * cqi)));
   const float yi = round_to<T>(sc * (zqi + (g.x * cqi + g.y * cqr)));
-  const float2 gn = make_float2(g.x * tr.ar - g.y * tr.ai, g.x * tr.ai + g.y * tr.ar);
+  const float2 gn = rotate(g, make_float2(tr.ar, tr.ai));
 
   if (!hok) return;  // nothing below reduces across lanes
   if (sub == 0) {

@@ -45,11 +45,6 @@ __device__ __forceinline__ float2 map_apply(float2 G, float2 s, float2 F) {
   const float im = IM_RE ? fmaf(G.y, s.x, G.x * s.y) : fmaf(G.x, s.y, G.y * s.x);
   return make_float2(re + F.x, im + F.y);
 }
-// G H, the product of two maps' rotations.
-__device__ __forceinline__ float2 map_product(float2 G, float2 H) {
-#pragma clang fp contract(off)
-  return make_float2(fmaf(G.x, H.x, -(G.y * H.y)), fmaf(G.x, H.y, G.y * H.x));
-}
 
 // Phase stamps of cdssm_fused_scan_fwd_stamped: segment entry, staging done,
 // local pass done, segment map published, look-back wait done, carry folded,
@@ -91,7 +86,7 @@ __device__ __forceinline__ void segment_carry(const OnePassBufs& ob, const float
     const float2 gu = make_float2(g.x, g.y);
 #pragma unroll
     for (int i = 0; i < EPT; ++i) segF[i] = map_apply<false>(gu, segF[i], Fx[u * SEGN + e0 + i]);
-    segG = map_product(gu, segG);
+    segG = rotate(gu, segG);
   }
   const int64_t sb0 = (int64_t(bi) * NSEG + seg) * H;  // (b, seg, head 0)
   unsigned long long* flag = ob.flag + sb0 + hbase;
@@ -153,7 +148,7 @@ __device__ __forceinline__ void segment_carry(const OnePassBufs& ob, const float
         const float2 gu = u < kFwdGroup - 1 ? G[u] : segG;
 #pragma unroll
         for (int i = 0; i < EPT; ++i) Fg[i] = map_apply<RE>(gu, Fg[i], u < kFwdGroup - 1 ? F[u][i] : segF[i]);
-        Gg = map_product(gu, Gg);
+        Gg = rotate(gu, Gg);
       }
       if (!okg) {
 #pragma unroll

@@ -250,6 +250,30 @@ def test_fused_token_kernel_matches_separate_kernels(dtype):
         assert rel(ca[-1]["scan"].state, cb[-1]["scan"].state) <= (1e-5 if dtype == torch.float32 else 2e-2)
 
 
+@pytest.mark.parametrize("dtype,head_dim", [(torch.float32, 64), (torch.float32, 128), (torch.bfloat16, 64),
+                                            (torch.bfloat16, 128)])
+def test_chunk_rotation_has_the_same_bits_on_every_route(dtype, head_dim):
+    """The chunk's running product of transitions (gam) after each token, from the tail, the token kernel and the
+    separate kernels: the transitions are the same values, so the product is the same bit for bit."""
+    from cdssm_hip.lm import CDSSMBlock, CDSSMConfig, CDSSMLMHeadModel, _clone_cache
+    torch.manual_seed(5)
+    m = CDSSMLMHeadModel(CDSSMConfig(d_model=128, n_layers=1, context_length=512, vocab_size=97, state_dim=2,
+                                     d_inner=8 * head_dim, head_dim=head_dim)).to(dtype).to(DEV).eval()
+    ids = torch.randint(0, 97, (6, 110), generator=torch.Generator().manual_seed(23)).to(DEV)
+    with torch.no_grad():
+        _, caches = m.prefill(ids[:, :100])
+        routes = {"tail": (True, True), "token": (True, False), "separate": (False, False)}
+        cs = {n: [_clone_cache(c) for c in caches] for n in routes}
+        try:
+            for t in range(100, 110):
+                for n, (CDSSMBlock.fused_step, CDSSMBlock.fused_tail) in routes.items():
+                    m.decode_step(ids[:, t], cs[n])
+                for n in ("token", "separate"):
+                    assert torch.equal(cs["tail"][0]["scan"].gam, cs[n][0]["scan"].gam), (n, t)
+        finally:
+            CDSSMBlock.fused_step = CDSSMBlock.fused_tail = True
+
+
 @pytest.mark.parametrize("dtype,d_inner", [(torch.float32, 512), (torch.bfloat16, 1024)])
 def test_fused_tail_matches_token_kernel_and_separate_epilogue(dtype, d_inner):
     """cdssm_decode_block_tail (token step + readout + GroupNorm step in one launch, one workgroup per batch
