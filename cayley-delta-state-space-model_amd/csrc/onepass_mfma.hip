@@ -32,9 +32,16 @@
 //  * sum_s x_s k_s: A = the coefficients (rows 4 h + part), B = K^T, which an
 //    MFMA against a selection matrix produces from the K fragments: its result
 //    layout, rounded back to bf16 (exact), is the B layout of 16x16x16.
-// fp32 operands (states, coefficients) enter as three bf16 terms, hi + mid +
-// lo = x to 2^-24 relative, so k.H and the updates keep fp32 accuracy; the
-// readouts q.H, q.c, whose result is rounded to bf16, take hi + mid (2^-16).
+//  * sum_s (q_t.k_s) x_s, both fp32: 4 x 1 by 1 x 4 fp32 products (4x4x1, 16 blocks), block = (head, 4
+//    tokens), whose results are the 4 sums of the lane's own token and head.
+// fp32 operands against K and Q (states, coefficients) enter as three bf16 terms,
+// hi + mid + lo = x to 2^-24 relative, so every sum keeps fp32 accuracy, the
+// readouts' too: y is the difference of a state's part and the part that erased
+// it, and where the two nearly cancel, operands of two terms (2^-16) leave
+// errors in its bf16 digits (D 64, a state 100 times the values written over
+// it: in a quarter of the outputs above 1e-3 of y's rounding, now in 1 in 300).
+// Holding that costs 0.6 to 3 us a call: B 8, H 16, L 4096, D 64 45.2 -> 46.4,
+// B 8, H 16, L 2048 29.9 -> 30.3; B 4, H 16, L 2048, D 128 71.3 -> 74.2.
 // Zeros times a non-finite value are not zero, so non-finite inputs are kept to their head and to the
 // tokens from theirs on: a block whose Gram sums are not finite zeroes the affected k slices, the tokens
 // with a non-finite k, write or beta enter the block with zero coefficients, and the head's state after the
@@ -73,7 +80,7 @@ struct MfCfg {
   static constexpr int SROW = 3 * D / 2 + 16;    // operand row, dwords: H | c | lo parts of D/2 each, and a pad
   static constexpr int OP = 16 * SROW + 64;      // 16 rows, 16 dwords apart per head (conflict-free writes)
   static constexpr int EB = 16 * 24;             // coefficient rows: 3 terms x 16 tokens bf16
-  static constexpr int ZERO = 24;                // zeros read by the lanes of the other heads
+  static constexpr int ZERO = 16 * (KS - 1) + 20;  // zeros, read in place of rows that do not take part
   static constexpr int NB(int Q) { return (Q + 15) / 16; }
   static constexpr int wave_dwords(int Q) { return NB(Q) * 64 * 8 + OP + EB; }
   static size_t lds_bytes(int Q) {
@@ -117,13 +124,6 @@ __device__ __forceinline__ void split3(float x0, float x1, uint32_t& hi, uint32_
   const uint32_t v0 = __float_as_uint(r0), v1 = __float_as_uint(r1);
   mid = __builtin_amdgcn_perm(v1, v0, 0x07060302u);
   lo = pack_bf16x2(r0 - __uint_as_float(v0 & 0xffff0000u), r1 - __uint_as_float(v1 & 0xffff0000u));
-}
-
-// x0, x1 as two bf16 terms (hi truncated, lo rounded; 2^-16 relative), packed in pairs.
-__device__ __forceinline__ void split_pair2(float x0, float x1, uint32_t& hi, uint32_t& lo) {
-  const uint32_t u0 = __float_as_uint(x0), u1 = __float_as_uint(x1);
-  hi = __builtin_amdgcn_perm(u1, u0, 0x07060302u);
-  lo = pack_bf16x2(x0 - __uint_as_float(u0 & 0xffff0000u), x1 - __uint_as_float(u1 & 0xffff0000u));
 }
 
 // The K or Q fragments of one block: head h, dims 32 ks + 8 (lane / 16) ..+8 of token lane % 16.
@@ -194,23 +194,39 @@ __device__ __forceinline__ void swap16(float& a, float& b) {
   b = __uint_as_float(s[1]);
 }
 
-// Tiles of 4 heads -> rows: lane (g, i) gets row[s] = tile_g[s][i] (s = 4 g' + r held by lane group g'),
-// zero where the mask (s < i, or s <= i with INCL) fails.
-template <bool INCL>
-__device__ __forceinline__ void mf_rows(f32x4_t (&t)[kMfHeads], int g, int i, float (&row)[16]) {
+// x[h] of lane group g' <-> x[g'] of lane group h
+__device__ __forceinline__ void mf_exchange(float (&x)[kMfHeads]) {
+  swap32(x[0], x[2]);
+  swap32(x[1], x[3]);
+  swap16(x[0], x[1]);
+  swap16(x[2], x[3]);
+}
+
+// Tiles of 4 heads -> rows: lane (g, i) gets row[s] = tile_g[s][i] (s = 4 g' + r held by lane group g') for
+// s < i, else zero.
+__device__ __forceinline__ void mf_rows(const f32x4_t (&t)[kMfHeads], int g, int i, float (&row)[16]) {
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    const bool keep = INCL ? 4 * g + r <= i : 4 * g + r < i;
     float x[kMfHeads];
 #pragma unroll
-    for (int h = 0; h < kMfHeads; ++h) x[h] = keep ? t[h][r] : 0.0f;
-    swap32(x[0], x[2]);
-    swap32(x[1], x[3]);
-    swap16(x[0], x[1]);
-    swap16(x[2], x[3]);
+    for (int h = 0; h < kMfHeads; ++h) x[h] = 4 * g + r < i ? t[h][r] : 0.0f;
+    mf_exchange(x);
 #pragma unroll
     for (int gp = 0; gp < 4; ++gp) row[4 * gp + r] = x[gp];
   }
+}
+
+// tile_g[i][i] for lane (g, i)
+__device__ __forceinline__ float mf_diag(const f32x4_t (&t)[kMfHeads], int g, int i) {
+  float x[kMfHeads];
+#pragma unroll
+  for (int h = 0; h < kMfHeads; ++h) {
+    x[h] = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) x[h] = 4 * g + r == i ? t[h][r] : x[h];
+  }
+  mf_exchange(x);
+  return (x[0] + x[1]) + (x[2] + x[3]);  // three zeros
 }
 
 // (I - L) x = x in place over the lane's 16-lane row, L strictly lower (row of this lane's token).
@@ -255,8 +271,8 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
   const bool hok = hv < H;
   const int hl = hok ? hv : H - 1;
 
-  // LDS: per wave the token slots (A: coefficient re, im, beta, sel; B: f re, im, a re, im), the operand
-  // rows and the coefficient rows; then the zeros, the chunk maps and the carry's buffers
+  // LDS: per wave the token slots (A: coefficient re, im, beta, sel, and in the correction pass a block's fp32
+  // coefficient rows; B: f re, im, a re, im), the operand rows and the coefficient rows; then the zeros, the chunk maps and the carry's buffers
   uint32_t* wl = mf_lds + wv * Cfg::wave_dwords(Q);
   float4* tokA = reinterpret_cast<float4*>(wl);
   float4* tokB = tokA + Cfg::NB(Q) * 64;
@@ -285,14 +301,11 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
   // row lane % 16 of head h's operand (the zeros where the row is another head's)
   uint32_t* opw = op + 4 * g * SROW + 16 * g + i;
   const uint32_t* opr = op + i * SROW + 16 * (i / 4) + 4 * g;
-  const uint32_t* ebr[kMfHeads];
+  const uint32_t* oprc = (i & 2) ? zero + 4 * g : opr + D;  // the lo part of c alone (rows 2, 3 hold H's there)
+  const uint32_t* ebr = eb + i * 24 + 2 * g;
   uint16_t* ebw = reinterpret_cast<uint16_t*>(eb) + 4 * g * 48 + i;
 #pragma unroll
-  for (int h = 0; h < kMfHeads; ++h) {
-    ebr[h] = i / 4 == h ? eb + i * 24 + 2 * g : zero;
-  }
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks) opw[2 * SROW + D + 16 * ks] = opw[3 * SROW + D + 16 * ks] = 0u;  // no lo part there
+  for (int ks = 0; ks < KS; ++ks) opw[2 * SROW + D + 16 * ks] = opw[3 * SROW + D + 16 * ks] = 0u;  // none in the local pass
   // selection operands: column n picks dim 2 n + u of a 32-dim step
   bf16x8_t sel2[2];
   {
@@ -400,22 +413,18 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
 
   f32x4_t st[KS][2];  // dims 32 ks + 2 i + u of head g: (H re, H im, c re, c im)
 
-  // the state into the operand rows: the local pass needs H in three terms (k.H), the correction pass c in
-  // three (k.c) and H in two (q.H)
+  // the state into the operand rows, hi in rows 0, 1 (re, im) and mid in rows 2, 3; the lo part of H in rows
+  // 0, 1 in the local pass, in rows 2, 3 in the correction pass, where rows 0, 1 hold c's
   auto put_state = [&](bool corr) {
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       uint32_t hi, mid, lo;
 #pragma unroll
       for (int p = 0; p < 2; ++p) {
-        if (!corr) {
-          split3(st[ks][0][p], st[ks][1][p], hi, mid, lo);
-          opw[p * SROW + D + 16 * ks] = lo;
-        } else {
-          split_pair2(st[ks][0][p], st[ks][1][p], hi, mid);
-        }
+        split3(st[ks][0][p], st[ks][1][p], hi, mid, lo);
         opw[p * SROW + 16 * ks] = hi;
         opw[(2 + p) * SROW + 16 * ks] = mid;
+        opw[(corr ? 2 + p : p) * SROW + D + 16 * ks] = lo;
       }
       if (corr) {
 #pragma unroll
@@ -476,12 +485,13 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
   };
   // the coefficient rows as A operands: e[p][m], term m (hi, mid, lo) of heads 2 p (k first half) and 2 p + 1
   auto load_coef = [&](bf16x8_t (&e)[kMfHeads / 2][3]) {
+    const int hi = opaque(i) / 4;
 #pragma unroll
     for (int p = 0; p < kMfHeads / 2; ++p)
 #pragma unroll
       for (int m = 0; m < 3; ++m) {
-        const uint2 x = *reinterpret_cast<const uint2*>(ebr[2 * p] + 8 * m);
-        const uint2 y = *reinterpret_cast<const uint2*>(ebr[2 * p + 1] + 8 * m);
+        const uint2 x = *reinterpret_cast<const uint2*>((hi == 2 * p ? ebr : zero) + 8 * m);
+        const uint2 y = *reinterpret_cast<const uint2*>((hi == 2 * p + 1 ? ebr : zero) + 8 * m);
         e[p][m] = __builtin_bit_cast(bf16x8_t, make_uint4(x.x, x.y, y.x, y.y));
       }
   };
@@ -566,7 +576,7 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
     if ((marked >> b) & 1u) bad = poison(ta);
     const float khr = MF_OWN(ka, 0) + MF_OWN(ka, 2), khi = MF_OWN(ka, 1) + MF_OWN(ka, 3);
     float Lr[16];
-    mf_rows<false>(gt, g, i, Lr);
+    mf_rows(gt, g, i, Lr);
 #pragma unroll
     for (int s = 0; s < 16; ++s) Lr[s] *= -ta.z;
     float xr, xi, cr, ci;  // the coefficient kept for the correction pass, and the state update's
@@ -637,29 +647,25 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
   clock(5);
 
   // ---- correction pass ----
-  // halves of a packed pair of rows (4 g + 2 p, 4 g + 2 p + 1) that are not column i's diagonal
-  uint32_t offdiag[2];
-#pragma unroll
-  for (int p = 0; p < 2; ++p)
-    offdiag[p] = (4 * g + 2 * p == i ? 0u : 0xffffu) | (4 * g + 2 * p + 1 == i ? 0u : 0xffff0000u);
   auto corr_block = [&](int b) {
-    f32x4_t gt[kMfHeads], pt[kMfHeads], ka[kMfHeads], qh[kMfHeads], qc[kMfHeads];
+    f32x4_t gt[kMfHeads], pt[kMfHeads], ka[kMfHeads], qh[kMfHeads], qc[kMfHeads], ql[kMfHeads];
     bf16x8_t kt[kMfHeads / 2][KS][2];
     bf16x8_t s1[KS], s2[KS], s3[KS];
     load_op(0, s1);
     load_op(D / 2, s2);
     load_op(D, s3);
-    float4 ta = tokA[b * 64 + lane];
-    const float4 tb = tokB[b * 64 + lane];
     const bool ex = (exact >> b) & 1u;
     // the three phases (q, k, the rest) are kept apart: interleaved, their tiles would not fit the registers
 #pragma unroll
-    for (int h = 0; h < kMfHeads; ++h) qh[h] = qc[h] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int h = 0; h < kMfHeads; ++h) qh[h] = qc[h] = ql[h] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     mf_gram<KS>(fk, fq, pt);
+    project(s3, fq, ql);
     project(s1, fq, qh);
+    const float qhr = MF_OWN(qh, 0) + (MF_OWN(qh, 2) + MF_OWN(ql, 2));
+    const float qhi = MF_OWN(qh, 1) + (MF_OWN(qh, 3) + MF_OWN(ql, 3));
+    __builtin_amdgcn_sched_barrier(0);
     project(s2, fq, qc);
-    const float qhr = MF_OWN(qh, 0) + MF_OWN(qh, 2), qhi = MF_OWN(qh, 1) + MF_OWN(qh, 3);
-    float qcr = MF_OWN(qc, 0) + MF_OWN(qc, 2), qci = MF_OWN(qc, 1) + MF_OWN(qc, 3);
+    float qcr = MF_OWN(qc, 0) + (MF_OWN(qc, 2) + MF_OWN(ql, 0)), qci = MF_OWN(qc, 1) + (MF_OWN(qc, 3) + MF_OWN(ql, 1));
     fq.load(qrs, voff(b + 1), hoff);
     __builtin_amdgcn_sched_barrier(0);
     for (int pass = 0;; ++pass) {
@@ -667,11 +673,15 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
       transpose_k(fk, kt);
 #pragma unroll
       for (int h = 0; h < kMfHeads; ++h) ka[h] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) s3[ks] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(oprc + 16 * ks));
       project(s2, fk, ka);
       project(s3, fk, ka);
       if (pass || mf_finite(gt)) break;
       mf_sanitize<KS>(fk, g, i);  // the local pass has marked the token
     }
+    float4 ta = tokA[b * 64 + lane];
+    const float4 tb = tokB[b * 64 + lane];
     fk.load(krs, voff(b + 1), hoff);
     __builtin_amdgcn_sched_barrier(0);
     uint32_t bad = 0;
@@ -682,7 +692,7 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
     float cxr = ta.z * (MF_OWN(ka, 0) + MF_OWN(ka, 2)), cxi = ta.z * (MF_OWN(ka, 1) + MF_OWN(ka, 3));
     {
       float Lr[16];
-      mf_rows<false>(gt, g, i, Lr);
+      mf_rows(gt, g, i, Lr);
 #pragma unroll
       for (int s = 0; s < 16; ++s) Lr[s] *= -ta.z;
       mf_solve(Lr, cxr, cxi);
@@ -699,51 +709,44 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
     put_coef(0, cr, ci);
     put_coef(2, -cxr, -cxi);
     wave_fence();
-    bf16x8_t e[kMfHeads / 2][3];
-    load_coef(e);
-    // sum_s P_ts (coefficients): P in two bf16 terms, rows s <= t for the local part, s < t for the
-    // correction's (whose readout is the one before the token); a head's sums in its own lane group
-    bf16x8_t ea[2];  // hi and mid, each against both terms of P
+    // sum_{s<t} P_ts (coefficient rows of s), in fp32: 16 products of 4 x 1 by 1 x 4 per step s, of which lane
+    // (g, i) gets the 4 sums of its own token and head; the coefficient rows pass through the block's slots
+    float* cf = reinterpret_cast<float*>(tokA + b * 64);
+    cf[64 * g + i] = ta.x;
+    cf[64 * g + 16 + i] = ta.y;
+    cf[64 * g + 32 + i] = -cxr;
+    cf[64 * g + 48 + i] = -cxi;
+    wave_fence();
+    float P[16];
+    mf_rows(pt, g, i, P);
+    const float pd = mf_diag(pt, g, i);
+    f32x4_t ps = {0.0f, 0.0f, 0.0f, 0.0f}, ps2 = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int m = 0; m < 2; ++m) {
-      const uint2 x = *reinterpret_cast<const uint2*>(eb + i * 24 + 2 * g + 8 * m);
-      ea[m] = __builtin_bit_cast(bf16x8_t, make_uint4(x.x, x.y, x.x, x.y));
+    for (int s = 0; s < 16; s += 4) {
+      const float4 x = *reinterpret_cast<const float4*>(cf + 64 * g + 16 * (i % 4) + s);
+      ps = __builtin_amdgcn_mfma_f32_4x4x1f32(x.x, P[s], ps, 0, 0, 0);
+      ps2 = __builtin_amdgcn_mfma_f32_4x4x1f32(x.y, P[s + 1], ps2, 0, 0, 0);
+      ps = __builtin_amdgcn_mfma_f32_4x4x1f32(x.z, P[s + 2], ps, 0, 0, 0);
+      ps2 = __builtin_amdgcn_mfma_f32_4x4x1f32(x.w, P[s + 3], ps2, 0, 0, 0);
     }
-    f32x4_t ri[kMfHeads], rx[kMfHeads];
-    const f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int h = 0; h < kMfHeads; ++h) {
-      uint32_t ph[2], pm[2];
-#pragma unroll
-      for (int p = 0; p < 2; ++p) {
-        const float x0 = 4 * g + 2 * p <= i ? pt[h][2 * p] : 0.0f, x1 = 4 * g + 2 * p + 1 <= i ? pt[h][2 * p + 1] : 0.0f;
-        split_pair2(x0, x1, ph[p], pm[p]);
-      }
-      const bf16x8_t bi = __builtin_bit_cast(bf16x8_t, make_uint4(ph[0], ph[1], pm[0], pm[1]));
-      const bf16x8_t bx = __builtin_bit_cast(bf16x8_t, make_uint4(ph[0] & offdiag[0], ph[1] & offdiag[1],
-                                                                 pm[0] & offdiag[0], pm[1] & offdiag[1]));
-      ri[h] = mfma16(ea[0], bi, z);
-      rx[h] = mfma16(ea[0], bx, z);
-      ri[h] = mfma16(ea[1], bi, ri[h]);
-      rx[h] = mfma16(ea[1], bx, rx[h]);
-    }
-    qcr += MF_OWN(rx, 2);
-    qci += MF_OWN(rx, 3);
+    ps += ps2;
+    qcr += ps[2];
+    qci += ps[3];
     float lr, li;
     if (!ex) {
-      const float vr = qhr + MF_OWN(ri, 0), vi = qhi + MF_OWN(ri, 1);
+      const float vr = qhr + fmaf(pd, ta.x, ps[0]), vi = qhi + fmaf(pd, ta.y, ps[1]);
       lr = tb.x * vr - tb.y * vi;
       li = tb.x * vi + tb.y * vr;
     } else {
-      float P[16], er = 0.0f, ei = 0.0f;
+      float er = 0.0f, ei = 0.0f;
       const int ii = opaque(i);
-      mf_rows<true>(pt, g, ii, P);
 #pragma unroll
       for (int s = 0; s < 16; ++s) {
         float nr = er, ni = ei;
         cmul_acc(nr, ni, row_bcast_dyn(tb.z, s), row_bcast_dyn(tb.w, s));
-        nr = fmaf(P[s], row_bcast_dyn(ta.x, s), nr);
-        ni = fmaf(P[s], row_bcast_dyn(ta.y, s), ni);
+        const float p = s == ii ? pd : P[s];
+        nr = fmaf(p, row_bcast_dyn(ta.x, s), nr);
+        ni = fmaf(p, row_bcast_dyn(ta.y, s), ni);
         er = s <= ii ? nr : er;
         ei = s <= ii ? ni : ei;
       }
@@ -751,12 +754,16 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
       li = fmaf(tb.x, qhi, fmaf(tb.y, qhr, ei));
       scale_local(f15r, f15i);
     }
+    bf16x8_t e[kMfHeads / 2][3];
+    load_coef(e);
     // g_{t-1} of the chunk
     float gr = row_shr<1>(tb.x, 1.0f), gi = row_shr<1>(tb.y, 0.0f);
     cmul_acc(gr, gi, Gr, Gi);
     const float yr = ta.w * fmaf(gr, qcr, fmaf(-gi, qci, lr)), yi = ta.w * fmaf(gr, qci, fmaf(gi, qcr, li));
-    if (hok && 16 * b + i < nt)
-      *reinterpret_cast<uint32_t*>(a.y + ((row0 + 16 * b + i) * H + hv) * 2) = pack_bf16x2(yr, yi);
+    if (hok && 16 * b + i < nt) {
+      char* yrow = reinterpret_cast<char*>(a.y + 2 * ((row0 + 16 * b) * H + hbase));  // the block's, wave-uniform
+      *reinterpret_cast<uint32_t*>(yrow + uint32_t(i * H + g) * 4u) = pack_bf16x2(yr, yi);
+    }
     if (b + 1 < nb) {
       update_state(e, kt);
       if (!ex) scale_local(f15r, f15i);

@@ -106,3 +106,37 @@ def test_continuing_call_after_a_four_launch_training_call():
         torch.cuda.synchronize()
         check_lookback()
         assert torch.equal(infer.y, y) and torch.equal(infer.h_final, h)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("source", ["carried", "written"])
+def test_a_large_state_that_is_overwritten_leaves_fp32_accuracy(source, D):
+    """Tokens with beta near 1 erase a state S times the values written over it, and the readout asks for the
+    direction just erased: y is what is left of two parts of size S.  Beside y's own rounding, half a bf16 ulp, its
+    error is that of fp32 sums of such parts, 2^-22 of their size (a few roundings of 2^-24; a state projects on a
+    direction with up to 4 S); operands of two bf16 terms would leave 2^-17.  alpha = omega = 0 and a small r, so that the transitions are 1 to 1e-7 and vp its clamp,
+    1e-3, and the dynamics' own error stays relative to y."""
+    log(f"[mfma forward] overwritten {source} D{D}")
+    B, H, L, S = 2, 5, 64, 100.0
+    g = torch.Generator().manual_seed(D)
+    n = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    unit = lambda x: x / x.norm(dim=-1, keepdim=True)  # noqa: E731
+    pool = unit(n(B, 1, H, 6, D)).expand(B, L, H, 6, D)
+    pick = lambda t: torch.gather(pool, 3, t[..., None, None].expand(B, L, H, 1, D))[:, :, :, 0]  # noqa: E731
+    ki = torch.randint(0, 6, (B, L, H), generator=g)
+    # the correction is read before the token's erasure, the local state after it
+    qi = torch.roll(ki, 1, 1) if source == "carried" else ki
+    size = torch.ones(L) if source == "carried" else torch.where(torch.arange(L) % 32 < 8, S, 1.0)
+    full = lambda v: torch.full((B, L, H), v)  # noqa: E731
+    x = dict(q=pick(qi), k=pick(ki), v=1e3 * n(B, L, H, 2) * size[:, None, None], beta=full(0.996), sel_C=full(1.0),
+             dt=full(0.5), r=full(0.05))
+    x = {name: t.to(torch.bfloat16).contiguous() for name, t in x.items()}
+    x.update(alpha=torch.zeros(H), omega=torch.zeros(H), c=4.0,
+             h0=S * n(B, H, 2, D) if source == "carried" else torch.zeros(B, H, 2, D))
+    y, h = run(to_dev(x))
+    yr, hr = oracle_fwd(x)
+    half_ulp = torch.exp2(yr.abs().clamp(min=1e-30).log2().floor() - 8)
+    over = ((y.double() - yr).abs() - half_ulp).clamp(min=0).max() / (4 * S)
+    log(f"   beyond y's rounding: {float(over):.1e} of the state")
+    assert float(over) <= 2.0 ** -22
+    assert rel(h, hr) <= TOL_H
