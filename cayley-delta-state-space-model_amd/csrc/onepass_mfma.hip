@@ -13,9 +13,9 @@
 //   x_t  =             beta_t (k_t.c) - beta_t sum_{s<t} (k_t.k_s) x_s     (c_{t+1} = c - sum_{s<=t} x_s k_s)
 //   y_t  = sel_t (f_t (q_t.H + sum_{s<=t} (q_t.k_s) x^_s) + g_{t-1} (q_t.c - sum_{s<t} (q_t.k_s) x_s))
 //   H'   = f_15 (H + sum_s x^_s k_s),   c' = c - sum_s x_s k_s
-// Where some |f_t| of the wave falls below kMfTiny (so 1 / f_t would overflow)
-// the block runs in true units: the same solve with the products of a carried
-// forward one step at a time, which never divides.
+// Where some quotient w_t / f_t of the wave would leave fp32's range (f_t near
+// its limits, or a large w_t) the block runs in true units: the same solve with
+// the products of a carried forward one step at a time, which never divides.
 //
 // A wave holds 4 heads of one chunk; a workgroup the 4 chunks of a segment.
 // Lane (g, i) = (lane / 16, lane % 16) owns token i of head g in the solve.
@@ -69,8 +69,11 @@ __global__ __launch_bounds__(64) void mf_epoch_kernel(unsigned long long* ctl) {
 }
 
 constexpr int kMfHeads = 4;            // heads per wave
-constexpr float kMfTiny = 0x1p-88f;    // |2^32 f|^2 below this (|f| < 2^-76): the block runs in true units
-constexpr float kMfScale = 0x1p32f;
+// A block runs in true units where some |2^60 f|^2 is below kMfTiny (|f| < 2^-112) or infinite, or some
+// quotient w / f not below kMfLarge (2^12 are left for the block's sums).
+constexpr float kMfTiny = 0x1p-104f;
+constexpr float kMfScale = 0x1p60f;
+constexpr float kMfLarge = 0x1p115f;
 
 typedef unsigned short u16x2_t __attribute__((ext_vector_type(2)));
 
@@ -395,10 +398,13 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
           row_cumprod(fr, fi);
           const float sr = fr * kMfScale, si = fi * kMfScale;
           const float m2 = sr * sr + si * si;
-          const bool ex = __builtin_amdgcn_ballot_w64(!(m2 >= kMfTiny)) != 0ull;
+          const float inv = __builtin_amdgcn_rcpf(m2);
+          float er = (wr * sr + wi * si) * inv * kMfScale, ei = (wi * sr - wr * si) * inv * kMfScale;
+          const bool out = !(m2 >= kMfTiny && m2 < __builtin_inff()) || !(fabsf(er) + fabsf(ei) < kMfLarge);
+          const bool ex = __builtin_amdgcn_ballot_w64(out) != 0ull;
           exact |= ex ? 1u << b : 0u;
-          const float inv = __builtin_amdgcn_rcpf(m2) * kMfScale;
-          const float er = ex ? wr : (wr * sr + wi * si) * inv, ei = ex ? wi : (wi * sr - wr * si) * inv;
+          er = ex ? wr : er;
+          ei = ex ? wi : ei;
           marked |= __builtin_amdgcn_ballot_w64(!((fabsf(er) + fabsf(ei)) + bt < __builtin_inff())) != 0ull ? 1u << b : 0u;
           tokA[b * 64 + lane] = make_float4(er, ei, bt, real ? ss[u] : 0.0f);
           tokB[b * 64 + lane] = make_float4(fr, fi, ar, ai);

@@ -140,3 +140,35 @@ def test_a_large_state_that_is_overwritten_leaves_fp32_accuracy(source, D):
     log(f"   beyond y's rounding: {float(over):.1e} of the state")
     assert float(over) <= 2.0 ** -22
     assert rel(h, hr) <= TOL_H
+
+
+def _flat_dynamics(H, E, c, cr):
+    """alpha, omega, c, and dt, r, for which every transition is real and |a| = E^(cr / 2)."""
+    ta = (1 - E ** 0.5) / (1 + E ** 0.5)  # ((1 - ta) / (1 + ta))^2 = E
+    return dict(alpha=torch.full((H,), 2 * ta), omega=torch.zeros(H), c=c), 1.0, cr / c
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("E,cr,size,L", [
+    (2.0 ** -9, 1.0, 2.0 ** 60, 130),   # |a| = 2^-4.5: 2^-72 over a block, under writes of 2^60
+    (2.0 ** -12, 1.0, 2.0 ** 100, 70),  # 2^-96 and 2^100
+    (2.0 ** -6, 1.0, 2.0 ** 90, 130),   # 2^-48 and 2^90
+    (2.0 ** -6, -0.9, 1e3, 24),         # |a| = 2^2.7: grows by 2^43 over a block
+])
+def test_writes_and_transitions_near_the_limits_stay_finite(D, E, cr, size, L):
+    """Quotients of a write and the block's product of transitions beyond fp32's range, with every value of the
+    recurrence inside it: those blocks run in true units.  The transitions' hardware exponentials are 2e-5 off, and
+    24 of them multiply where they grow."""
+    log(f"[mfma forward] limits D{D} E{E:.1e} cr{cr} size{size:.0e} L{L}")
+    B, H = 2, 6
+    rates, dt, r = _flat_dynamics(H, E, 4.0, cr)
+    x = draw_inputs(ScanConfig("t", B=B, H=H, L=L, D=D), seed=7)
+    x.update(rates, v=x["v"] * size, dt=torch.full_like(x["dt"], dt), r=torch.full_like(x["r"], r), h0=None)
+    x = {k: v for k, v in x.items() if v is not None}
+    if cr < 0:
+        x["v"][:, :12] = 0  # what is written last in the first block, where the product is largest, decides
+    y, h = run(to_dev(x))
+    yr, hr = oracle_fwd(x)
+    assert y.isfinite().all() and h.isfinite().all()
+    tol = 24 * 2e-5 if cr < 0 else 0.0
+    assert rel(y, yr) <= TOL_Y + tol and rel(h, hr) <= TOL_H + tol, (rel(y, yr), rel(h, hr))
