@@ -12,10 +12,14 @@
 //   x^_t = w_t / f_t - beta_t (k_t.H) - beta_t sum_{s<t} (k_t.k_s) x^_s    (update coefficients, z_t = f_t (H + sum_{s<=t} x^_s k_s))
 //   x_t  =             beta_t (k_t.c) - beta_t sum_{s<t} (k_t.k_s) x_s     (c_{t+1} = c - sum_{s<=t} x_s k_s)
 //   y_t  = sel_t (f_t (q_t.H + sum_{s<=t} (q_t.k_s) x^_s) + g_{t-1} (q_t.c - sum_{s<t} (q_t.k_s) x_s))
-//   H'   = f_15 (H + sum_s x^_s k_s),   c' = c - sum_s x_s k_s
-// Where some quotient w_t / f_t of the wave would leave fp32's range (f_t near
-// its limits, or a large w_t) the block runs in true units: the same solve with
-// the products of a carried forward one step at a time, which never divides.
+//   H'   = f_15 H + sum_s (f_15 x^_s) k_s,   c' = c - sum_s x_s k_s
+// A head whose quotients w_t / f_t would leave fp32's range (f_t near its limits,
+// or a large w_t) runs its block in true units: the same solve with the products
+// of a carried forward one step at a time, which never divides.  That is decided
+// per head, and nothing else crosses heads, so a head's bits do not depend on the
+// others of its wave.  With |f| down to 2^-112 in the quotients one block in 20 of
+// a drawn call at B 8, H 16, L 4096 is such a one for some head of its wave (one
+// in 5 at 2^-76); if all are, the call takes 48.7 in place of 42.2 us.
 //
 // A wave holds 4 heads of one chunk; a workgroup the 4 chunks of a segment.
 // Lane (g, i) = (lane / 16, lane % 16) owns token i of head g in the solve.
@@ -38,10 +42,12 @@
 // hi + mid + lo = x to 2^-24 relative, so every sum keeps fp32 accuracy, the
 // readouts' too: y is the difference of a state's part and the part that erased
 // it, and where the two nearly cancel, operands of two terms (2^-16) leave
-// errors in its bf16 digits (D 64, a state 100 times the values written over
-// it: in a quarter of the outputs above 1e-3 of y's rounding, now in 1 in 300).
-// Holding that costs 0.6 to 3 us a call: B 8, H 16, L 4096, D 64 45.2 -> 46.4,
-// B 8, H 16, L 2048 29.9 -> 30.3; B 4, H 16, L 2048, D 128 71.3 -> 74.2.
+// errors in its bf16 digits (D 64, a state 100 times the values written over it:
+// above 1e-3 of y's rounding in a quarter of the outputs, now in 1 in 300).
+// us per call with two terms / now: B 8, H 16, L 4096, D 64 45.2 / 44.9, L 2048
+// 29.9 / 29.4, B 1, H 4, L 512 22.8 / 23.4; D 128, B 4, H 16, L 2048 71.3 / 69.6.
+// The third term cost 0.4 to 3 us of it; scaling the state and the coefficients
+// ahead of the update, not the sum after it, gave that back.
 // Zeros times a non-finite value are not zero, so non-finite inputs are kept to their head and to the
 // tokens from theirs on: a block whose Gram sums are not finite zeroes the affected k slices, the tokens
 // with a non-finite k, write or beta enter the block with zero coefficients, and the head's state after the
@@ -69,7 +75,7 @@ __global__ __launch_bounds__(64) void mf_epoch_kernel(unsigned long long* ctl) {
 }
 
 constexpr int kMfHeads = 4;            // heads per wave
-// A block runs in true units where some |2^60 f|^2 is below kMfTiny (|f| < 2^-112) or infinite, or some
+// A head's block runs in true units where some |2^60 f|^2 is below kMfTiny (|f| < 2^-112) or infinite, or some
 // quotient w / f not below kMfLarge (2^12 are left for the block's sums).
 constexpr float kMfTiny = 0x1p-104f;
 constexpr float kMfScale = 0x1p60f;
@@ -324,7 +330,9 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
   MfFrags<KS> fk, fq;  // the current block's K and Q fragments
 
   // ---- staging: lane (g, i) computes token i of each block for its head ----
-  uint32_t exact = 0, marked = 0;  // bit b: block b runs in true units; holds a non-finite coefficient, beta or k
+  // bit 4 b + h: block b of head h runs in true units (at most 8 blocks); bit b: block b holds a non-finite
+  // coefficient, beta or k
+  uint32_t exact = 0, marked = 0;
   float Gr = 1.0f, Gi = 0.0f;
   if (live) {
     const float al = a.alpha[hl], om = a.omega[hl];
@@ -401,10 +409,17 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
           const float inv = __builtin_amdgcn_rcpf(m2);
           float er = (wr * sr + wi * si) * inv * kMfScale, ei = (wi * sr - wr * si) * inv * kMfScale;
           const bool out = !(m2 >= kMfTiny && m2 < __builtin_inff()) || !(fabsf(er) + fabsf(ei) < kMfLarge);
-          const bool ex = __builtin_amdgcn_ballot_w64(out) != 0ull;
-          exact |= ex ? 1u << b : 0u;
-          er = ex ? wr : er;
-          ei = ex ? wi : ei;
+          const unsigned long long m = __builtin_amdgcn_ballot_w64(out);
+          if (m) {
+            uint32_t heads = 0;
+#pragma unroll
+            for (int h = 0; h < kMfHeads; ++h) heads |= ((m >> (16 * h)) & 0xffffull) ? 1u << h : 0u;
+            exact |= heads << (kMfHeads * b);
+            if ((heads >> opaque(g)) & 1u) {
+              er = wr;
+              ei = wi;
+            }
+          }
           marked |= __builtin_amdgcn_ballot_w64(!((fabsf(er) + fabsf(ei)) + bt < __builtin_inff())) != 0ull ? 1u << b : 0u;
           tokA[b * 64 + lane] = make_float4(er, ei, bt, real ? ss[u] : 0.0f);
           tokB[b * 64 + lane] = make_float4(fr, fi, ar, ai);
@@ -547,6 +562,7 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
     xi = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(ai), 0x101, 0xF, 0xF, false));
   };
   const float qnan = __builtin_nanf("");
+  auto mine = [&](int b) { return ((exact >> (kMfHeads * b)) >> opaque(g)) & 1u; };  // this lane's head in true units
   // Tokens of a marked block (bit t) whose coefficient or beta is not finite in this lane's head; their
   // coefficient and beta are replaced by zeros.
   auto poison = [&](float4& ta) {
@@ -585,44 +601,45 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
     mf_rows(gt, g, i, Lr);
 #pragma unroll
     for (int s = 0; s < 16; ++s) Lr[s] *= -ta.z;
-    float xr, xi, cr, ci;  // the coefficient kept for the correction pass, and the state update's
-    const bool ex = (exact >> b) & 1u;
+    const bool ex = (exact >> (kMfHeads * b)) & 15u;
     float f15r = row_bcast<15>(tb.x);
     const float f15i = row_bcast<15>(tb.y);
     if (bad) f15r = qnan;  // the state after the block
-    if (!ex) {
-      xr = fmaf(-ta.z, khr, ta.x);
-      xi = fmaf(-ta.z, khi, ta.y);
-      mf_solve(Lr, xr, xi);
-      cr = xr;
-      ci = xi;
-    } else {
+    scale_local(f15r, f15i);
+    float xr = fmaf(-ta.z, khr, ta.x), xi = fmaf(-ta.z, khi, ta.y);
+    mf_solve(Lr, xr, xi);
+    float cr = f15r, ci = f15i;  // to the block's end
+    if (ex) {
+      asm volatile("");  // a branch, not selects
       // e_t = w_t - beta_t f_t (k_t.H) + a_t A_t, A_t = sum_{s<t} prod_{s<u<t} a_u L_ts e_s
       const float br = ta.x - ta.z * (tb.x * khr - tb.y * khi), bi2 = ta.y - ta.z * (tb.x * khi + tb.y * khr);
-      float Ar = 0.0f, Ai = 0.0f;
+      float Ar = 0.0f, Ai = 0.0f, tr = 0.0f, ti = 0.0f;
       const int ii = opaque(i);
-      xr = xi = 0.0f;
 #pragma unroll
       for (int s = 0; s < 16; ++s) {
         const float er = br + (tb.z * Ar - tb.w * Ai), ei = bi2 + (tb.z * Ai + tb.w * Ar);
-        xr = s == ii ? er : xr;
-        xi = s == ii ? ei : xi;
+        tr = s == ii ? er : tr;
+        ti = s == ii ? ei : ti;
         const float sr = row_bcast_dyn(tb.z, s), si = row_bcast_dyn(tb.w, s);
         cmul_acc(Ar, Ai, sr, si);
         Ar = fmaf(Lr[s], row_bcast_dyn(er, s), Ar);
         Ai = fmaf(Lr[s], row_bcast_dyn(ei, s), Ai);
       }
-      suffix(tb.z, tb.w, cr, ci);
-      cmul_acc(cr, ci, xr, xi);
-      scale_local(f15r, f15i);
+      float ur, ui;
+      suffix(tb.z, tb.w, ur, ui);
+      const bool m = mine(b);
+      xr = m ? tr : xr;
+      xi = m ? ti : xi;
+      cr = m ? ur : cr;
+      ci = m ? ui : ci;
     }
+    cmul_acc(cr, ci, xr, xi);
     tokA[b * 64 + lane] = make_float4((bad >> i) & 1u ? qnan : xr, xi, ta.z, ta.w);
     put_coef(0, cr, ci);
     wave_fence();
     bf16x8_t e[kMfHeads / 2][3];
     load_coef(e);
     update_state(e, kt);
-    if (!ex) scale_local(f15r, f15i);
     if (b + 1 < nb) put_state(false);
     wave_fence();
   };
@@ -653,6 +670,7 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
   clock(5);
 
   // ---- correction pass ----
+  char* yblk = reinterpret_cast<char*>(a.y) + (row0 * H + hbase) * 4;  // the block's rows
   auto corr_block = [&](int b) {
     f32x4_t gt[kMfHeads], pt[kMfHeads], ka[kMfHeads], qh[kMfHeads], qc[kMfHeads], ql[kMfHeads];
     bf16x8_t kt[kMfHeads / 2][KS][2];
@@ -660,7 +678,7 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
     load_op(0, s1);
     load_op(D / 2, s2);
     load_op(D, s3);
-    const bool ex = (exact >> b) & 1u;
+    const bool ex = (exact >> (kMfHeads * b)) & 15u;
     // the three phases (q, k, the rest) are kept apart: interleaved, their tiles would not fit the registers
 #pragma unroll
     for (int h = 0; h < kMfHeads; ++h) qh[h] = qc[h] = ql[h] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
@@ -706,12 +724,16 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
     float f15r = row_bcast<15>(tb.x);
     const float f15i = row_bcast<15>(tb.y);
     if (bad) f15r = qnan;  // the local state, and through the product of a every later output of the chunk
-    float cr = ta.x, ci = ta.y;
+    float cr = f15r, ci = f15i;
     if (ex) {
       asm volatile("");  // a branch, not selects
-      suffix(tb.z, tb.w, cr, ci);
-      cmul_acc(cr, ci, ta.x, ta.y);
+      float ur, ui;
+      suffix(tb.z, tb.w, ur, ui);
+      const bool m = mine(b);
+      cr = m ? ur : cr;
+      ci = m ? ui : ci;
     }
+    cmul_acc(cr, ci, ta.x, ta.y);
     put_coef(0, cr, ci);
     put_coef(2, -cxr, -cxi);
     wave_fence();
@@ -738,12 +760,10 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
     ps += ps2;
     qcr += ps[2];
     qci += ps[3];
-    float lr, li;
-    if (!ex) {
-      const float vr = qhr + fmaf(pd, ta.x, ps[0]), vi = qhi + fmaf(pd, ta.y, ps[1]);
-      lr = tb.x * vr - tb.y * vi;
-      li = tb.x * vi + tb.y * vr;
-    } else {
+    const float vr = qhr + fmaf(pd, ta.x, ps[0]), vi = qhi + fmaf(pd, ta.y, ps[1]);
+    float lr = tb.x * vr - tb.y * vi, li = tb.x * vi + tb.y * vr;
+    if (ex) {
+      asm volatile("");
       float er = 0.0f, ei = 0.0f;
       const int ii = opaque(i);
 #pragma unroll
@@ -756,9 +776,10 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
         er = s <= ii ? nr : er;
         ei = s <= ii ? ni : ei;
       }
-      lr = fmaf(tb.x, qhr, fmaf(-tb.y, qhi, er));
-      li = fmaf(tb.x, qhi, fmaf(tb.y, qhr, ei));
-      scale_local(f15r, f15i);
+      if (mine(b)) {
+        lr = fmaf(tb.x, qhr, fmaf(-tb.y, qhi, er));
+        li = fmaf(tb.x, qhi, fmaf(tb.y, qhr, ei));
+      }
     }
     bf16x8_t e[kMfHeads / 2][3];
     load_coef(e);
@@ -766,13 +787,10 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
     float gr = row_shr<1>(tb.x, 1.0f), gi = row_shr<1>(tb.y, 0.0f);
     cmul_acc(gr, gi, Gr, Gi);
     const float yr = ta.w * fmaf(gr, qcr, fmaf(-gi, qci, lr)), yi = ta.w * fmaf(gr, qci, fmaf(gi, qcr, li));
-    if (hok && 16 * b + i < nt) {
-      char* yrow = reinterpret_cast<char*>(a.y + 2 * ((row0 + 16 * b) * H + hbase));  // the block's, wave-uniform
-      *reinterpret_cast<uint32_t*>(yrow + uint32_t(i * H + g) * 4u) = pack_bf16x2(yr, yi);
-    }
+    if (hok && 16 * b + i < nt) *reinterpret_cast<uint32_t*>(yblk + uint32_t(i * H + g) * 4u) = pack_bf16x2(yr, yi);
     if (b + 1 < nb) {
+      scale_local(f15r, f15i);
       update_state(e, kt);
-      if (!ex) scale_local(f15r, f15i);
       put_state(true);
       wave_fence();
       cmul_acc(Gr, Gi, f15r, f15i);
@@ -800,7 +818,10 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
     Gr = 1.0f;
     Gi = 0.0f;
 #pragma unroll 1
-    for (int b = 0; b < nb; ++b) corr_block(b);
+    for (int b = 0; b < nb; ++b) {
+      corr_block(b);
+      yblk += 64 * H;
+    }
   }
   clock(6);
   if (stamping && lane == 0) {

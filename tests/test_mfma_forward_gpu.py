@@ -172,3 +172,40 @@ def test_writes_and_transitions_near_the_limits_stay_finite(D, E, cr, size, L):
     assert y.isfinite().all() and h.isfinite().all()
     tol = 24 * 2e-5 if cr < 0 else 0.0
     assert rel(y, yr) <= TOL_Y + tol and rel(h, hr) <= TOL_H + tol, (rel(y, yr), rel(h, hr))
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_a_heads_bits_do_not_depend_on_the_others_of_its_wave(D):
+    """Heads beside one that decays fast, so that its blocks run in true units, or that holds a NaN in its last
+    block: the same bits as beside an ordinary one."""
+    log(f"[mfma forward] neighbours D{D}")
+    x = to_dev(draw_inputs(ScanConfig("t", B=2, H=8, L=333, D=D, h0_std=0.1), seed=11))
+    ref = run(x)
+    rest = [0, 1, 3, 4, 5, 7]
+    for change in ("decay", "dt", "k", "h0"):
+        z = {n: (t.clone() if isinstance(t, torch.Tensor) else t) for n, t in x.items()}
+        if change == "decay":
+            z["alpha"][[2, 6]] = 12.0
+        elif change == "h0":
+            z["h0"][:, [2, 6], 0, 3] = float("nan")
+        else:
+            z[change][:, 330, [2, 6]] = float("nan")
+        y, h = run(z)
+        assert torch.equal(y[:, :, rest], ref[0][:, :, rest]) and torch.equal(h[:, rest], ref[1][:, rest]), change
+        assert not torch.equal(h[:, [2, 6]], ref[1][:, [2, 6]]), change
+
+
+@pytest.mark.parametrize("name", ["beta", "k", "v"])
+def test_non_finite_input_in_two_heads_of_a_wave(name):
+    """Head 0 at token 20, head 3 at token 100, of one wave: each is clean before its token and not finite from it
+    on, and the other heads are a clean run's."""
+    x = to_dev(draw_inputs(ScanConfig("t", B=1, H=5, L=150, D=64), seed=5))
+    y0, h0 = run(x)
+    x[name] = x[name].clone()
+    for h, t in ((0, 20), (3, 100)):
+        x[name][0, t, h] = float("inf")
+    y1, h1 = run(x)
+    assert torch.equal(y0[:, :, [1, 2, 4]], y1[:, :, [1, 2, 4]]) and torch.equal(h0[:, [1, 2, 4]], h1[:, [1, 2, 4]])
+    for h, t in ((0, 20), (3, 100)):
+        assert torch.equal(y0[:, :t, h], y1[:, :t, h])
+        assert not y1[:, t:, h].isfinite().any() and not h1[:, h].isfinite().any()
