@@ -109,6 +109,7 @@ struct MfArgs {
   int L, H, Q, NC, NSEG, B, n_hg;
   bool wide;  // 8-byte loads of the per-token scalars
   unsigned long long* stamps;
+  int stamp_heads;  // heads to a stamp record's item
 };
 
 // LDS handed between lanes of one wave: the wave's LDS accesses complete in
@@ -826,9 +827,11 @@ __device__ __forceinline__ void mf_segment(const MfArgs& a, int idx, unsigned lo
   clock(6);
   if (stamping && lane == 0) {
     clock(7);
-    unsigned long long* o = a.stamps + (int64_t(idx) * W + wv) * kStampPoints;
+    const int n_hg = (H + a.stamp_heads - 1) / a.stamp_heads, sg = hbase / a.stamp_heads;
+    unsigned long long* o = a.stamps + (((int64_t(seg) * a.B + bi) * n_hg + sg) * W + wv) * kStampPoints;
+    if (sg * a.stamp_heads == hbase)
 #pragma unroll
-    for (int n = 0; n < kStampPoints; ++n) o[n] = ts[n];
+      for (int n = 0; n < kStampPoints; ++n) o[n] = ts[n];
   }
 }
 
@@ -881,10 +884,14 @@ int mf_launch(const MfmaForward& p, hipStream_t stream, hipEvent_t* ev) {
   a.wide = p.H % kMfHeads == 0 && on(p.beta, 8) && on(p.sel_c, 8) && on(p.dt, 8) && on(p.r, 8) && on(p.v, 4);
   const int64_t items = int64_t(w.NSEG) * p.B * a.n_hg;
   a.stamps = nullptr;
+  a.stamp_heads = kMfHeads;
   if (p.stamps) {
-    if (p.stamps_len < items * kOnePassW * kStampPoints) {
-      cdssm_host::set_error("cdssm_fused_scan_fwd_stamped: %lld stamp words needed (%lld given)",
-                            (long long)(items * kOnePassW * kStampPoints), (long long)p.stamps_len);
+    // a buffer for items of 8 heads (the sequential kernel's) takes the records of each one's first 4
+    if (p.stamps_len < items * kOnePassW * kStampPoints && D == 64) a.stamp_heads = 2 * kMfHeads;
+    const int64_t words = int64_t(w.NSEG) * p.B * ((p.H + a.stamp_heads - 1) / a.stamp_heads) * kOnePassW * kStampPoints;
+    if (p.stamps_len < words) {
+      cdssm_host::set_error("cdssm_fused_scan_fwd_stamped: %lld stamp words needed (%lld given)", (long long)words,
+                            (long long)p.stamps_len);
       return CDSSM_EINVAL;
     }
     a.stamps = p.stamps;

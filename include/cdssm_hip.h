@@ -323,10 +323,14 @@ int cdssm_fused_scan_bwd_profile(int dtype, const void* q, const void* k, const 
  * staging done, local pass done, segment map published, look-back wait done,
  * carry folded, correction pass done, segment end.  stamps: device memory of
  * stamps_len 8-byte words; word ((item * 4 + wave) * 8 + point) for wave
- * 0..3 of the workgroup of item = segment * B * n_hg + b * n_hg + head group
- * (n_hg = ceil(H / 8) head groups for bf16 D = 64, the same layout for the
- * other instances with their heads per wave); the caller clears the buffer to
- * tell unwritten records.
+ * 0..3 of the workgroup of item = segment * B * n_hg + b * n_hg + head group,
+ * n_hg = ceil(H / heads per wave); the caller clears the buffer to tell
+ * unwritten records.  Heads per wave: 4 in the matrix-core forward; in the
+ * sequential one for bf16 D = 64 8, or 4 where H > 4 and the items of 8 heads
+ * are fewer than the compute units; 4 for bf16 D = 128 and fp32 D = 64; 2 for
+ * fp32 D = 128.  (n_hg = H always suffices.)  With a buffer that holds only
+ * the layout of 8 heads the matrix-core forward writes that one, from the
+ * waves of each item's first 4 heads.
  * Returns -1 (nothing launched) if the buffer holds fewer than
  * items * 32 words or the shape takes the four-launch forward.  Results are
  * bit-identical to cdssm_fused_scan_fwd.

@@ -107,3 +107,37 @@ def test_stamped_backward_equals_plain_backward_and_records_every_wave(name, B, 
     # one main-pass wave per (b, chunk, head group): head groups divide H
     assert (B * nc * H) % main.shape[0] == 0, (main.shape, B, nc, H)
     log(f"   {corr.shape[0]} correction-pass and {main.shape[0]} main-pass wave records, points in order")
+
+
+@pytest.mark.parametrize("B,H,L,D,heads", [(4, 16, 3904, 64, 4), (4, 16, 3904, 64, 8), (3, 6, 3000, 64, 4),
+                                           (2, 10, 3700, 128, 4)])
+def test_stamps_of_the_matrix_core_forward_lie_where_documented(B, H, L, D, heads):
+    """The inference forward's default kernel at these shapes: a buffer of exactly the documented words, one record per
+    wave at item = (segment * B + b) * n_hg + head group (with the layout of 8 heads, of each item's first 4 heads).
+    By the records at those places, the waves that the last segment has no chunk for stage nothing (the loads take
+    the others over 1 us), and a segment's look-back wait ends after the previous segment of its row and heads has
+    made its map.  The call's outputs are a plain call's."""
+    from cdssm_hip import _lib
+    log(f"[phase stamps] matrix cores: B{B} H{H} L{L} D{D}, {heads} heads to an item")
+    pf = _prepared(ScanConfig("s", B=B, H=H, L=L, D=D, h0_std=0.1))
+    pf()
+    torch.cuda.synchronize()
+    y, hf = pf.y.clone(), pf.h_final.clone()
+    nseg, n_hg = -(-L // (4 * D)), -(-H // heads)
+    words = nseg * B * n_hg * 32
+    guard = torch.zeros(words + 64, dtype=torch.int64, device=DEV)
+    call = lambda n: pf._lib.cdssm_fused_scan_fwd_stamped(*pf._args, _lib.ptr(guard), n, _lib.stream_of(DEV))  # noqa: E731
+    assert call(words if heads == 4 else words + 1) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(pf.y, y) and torch.equal(pf.h_final, hf)
+    st = guard.cpu()
+    assert not st[words:].any()
+    st = st[:words].view(nseg, B, n_hg, 4, 8)
+    live = torch.arange(nseg * 4).view(nseg, 1, 1, 4).expand(nseg, B, n_hg, 4) < -(-L // D)
+    assert bool((st[..., 0] > 0).all()) and bool((st[..., 1:] >= st[..., :-1])[live].all())
+    staging = st[..., 1] - st[..., 0]
+    log(f"   staging: {int(staging[live].min())} ticks and more, {int(staging[~live].max())} and less without a chunk")
+    assert int(staging[live].min()) > int(staging[~live].max())
+    assert bool((st[1:, ..., 0, 4] >= st[:-1, ..., 0, 2]).all()), "a wait ended before the map it waits for was there"
+    if heads == 8:
+        assert call(words - 1) == -1 and "stamp words needed" in _lib.last_error()
