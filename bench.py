@@ -829,6 +829,7 @@ def main():
         return
 
     import torch
+    from cdssm_hip import _lib
     from cdssm_hip.scan import PreparedForward, set_forward_path
     from cdssm_hip.workloads import CONFIGS, draw_inputs, scan_bytes
 
@@ -892,11 +893,7 @@ def main():
     phases = run.profile(args.steps)
     main_ms = phases["main"]
     one_pass = all(phases[k] == 0.0 for k in ("summary", "carry_fold", "carry_replay"))
-    # one launch: on the matrix cores where one round of workgroups (two per CU at D = 64, one at 128) takes
-    # every segment of 4 chunks and 4 heads, else the sequential kernel
-    n_cu = torch.cuda.get_device_properties(dev).multi_processor_count
-    items = cfg.B * -(-cfg.L // (4 * cfg.D)) * -(-cfg.H // 4)
-    matrix = args.forward_path == "auto" and items <= n_cu * (2 if cfg.D == 64 else 1)
+    matrix = _lib.load().cdssm_fused_scan_fwd_matrix_cores(1, cfg.B, cfg.L, cfg.H, cfg.D, cfg.N, cfg.D) == 1
     kernel = ("mf_onepass_kernel" if matrix else "fused_fwd_onepass_kernel") if one_pass else "fused_fwd_main_kernel"
     traffic_file = TRAFFIC_FILES[kernel]
 

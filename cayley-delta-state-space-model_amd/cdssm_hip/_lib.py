@@ -59,6 +59,7 @@ SIGNATURES = {
     "cdssm_fused_scan_bwd_profile": (_I32, [_I32, _P, _P, _P, _P, _P, _P, _P, _P, _P, _F32, _P, _P, _P,
                                             _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P,
                                             _I64, _I64, _I64, _I64, _I64, _I64, _P, _I32, _P]),
+    "cdssm_fused_scan_fwd_matrix_cores": (_I32, [_I32] + [_I64] * 6),
     "cdssm_fused_scan_fwd_abar": (_I32, [_I32] + [_P] * 11 + [_I64] * 6 + [_P]),
     "cdssm_fused_scan_fwd_abar_train": (_I32, [_I32] + [_P] * 11 + [_I64] * 6 + [_P]),
     "cdssm_fused_scan_bwd_abar": (_I32, [_I32] + [_P] * 19 + [_I64] * 6 + [_P]),

@@ -1777,6 +1777,18 @@ namespace {
 // workspace NULL, the library's static per-device scratch (inference only).
 int scratch_regions(const FwdLayout& w, FwdRegions* reg);
 
+// Whether an inference forward on scan-level inputs runs the matrix-core kernel: bf16, and one round of
+// resident workgroups (2 per CU at D = 64, 1 at D = 128) takes every segment.  Measured on MI355X against the
+// better of the other two forms, us per call: D 64 H4 L512 41.3 -> 23.4, B8 H16 L2048 39 -> 29.4, B8 H16 L4096
+// (the largest single round) 48.9 -> 44.9; D 128 B4 H16 L2048 74.8 -> 69.6, B1 H16 L8192 76.5 -> 71.8; with
+// more rounds it is the slower one (B1 H32 L65536 D64: 177 against 196, looping over segments).  The
+// gate-level form keeps the sequential kernel: a model's prefill feeds decode states whose bits a
+// generation continues from, and 24 bf16 layers turn another order of sums into 1e-2 of those states.
+bool takes_matrix_cores(int dtype, int64_t B, int64_t L, int64_t H, int64_t D, int64_t chunk) {
+  return dtype == 1 && cdssm_host::scan_path() == cdssm_host::kPathAuto &&
+         mfma_forward_fits(B, L, H, int(D), int(chunk));
+}
+
 int fused_fwd_entry(int dtype, const void* q, const void* k, const void* v, const void* beta,
                     const void* sel_c, const void* dt, const void* r, const float* alpha,
                     const float* omega, float c, const float* h0, void* y, float* h_final,
@@ -1853,15 +1865,7 @@ int fused_fwd_entry(int dtype, const void* q, const void* k, const void* v, cons
     reg = full_regions(workspace, lay);
   }
   const int b = int(B), l = int(L), hh = int(H), qc = int(chunk);
-  // bf16 scan-level inference: the matrix-core one-launch forward, where one round of resident
-  // workgroups (2 per CU at D = 64, 1 at D = 128) takes every segment.  Measured on MI355X against the
-  // better of the other two forms: D 64 H4 L512 39.6 -> 23.0 us, B8 H16 L2048 35.2 -> 28.1, B8 H16 L4096
-  // (the largest single round) 43.4 -> 41.7; D 128 B4 H16 L2048 72.1 -> 65.2, L8192 94.0 -> 76.1; with
-  // more rounds it is the slower one (B1 H32 L65536 D64: 177 against 196 us, looping over segments).  The
-  // gate-level form keeps the sequential kernel: a model's prefill feeds decode states whose bits a
-  // generation continues from, and 24 bf16 layers turn another order of sums into 1e-2 of those states
-  if (dtype == 1 && !ssd && !abar && !save && cdssm_host::scan_path() == cdssm_host::kPathAuto &&
-      mfma_forward_fits(B, L, H, int(D), qc)) {
+  if (!ssd && !abar && !save && takes_matrix_cores(dtype, B, L, H, D, chunk)) {
     if (path) *path = cdssm_host::kPathOne;
     return launch_mfma_forward(MfmaForward{q, k, v, beta, sel_c, dt, r, alpha, omega, c, h0, y, h_final, reg.onepass, b,
                                            l, hh, int(D), qc, cont, t_stamps.buf, t_stamps.len},
@@ -1893,8 +1897,9 @@ int fused_fwd_entry(int dtype, const void* q, const void* k, const void* v, cons
     return launch_fused_fwd<ABar<F32>, 128, 32, 32>(CDSSM_FWD_ARGS, rr);
   }
   if (dtype == 1) {
-    // the training forward takes the same layout as the inference forward of the
-    // shape (its workspace does not depend on it), so the two stay bit-identical
+    // the training forward takes the same layout as the sequential inference forward of the shape (its
+    // workspace does not depend on it), so those two are bit-identical; where the inference forward takes the
+    // matrix cores its sums have another order
     if (D == 64 && fill_with_4_heads_per_wave(B, L, H, chunk))
       return launch_fused_fwd<BF16, 64, 16, CDSSM_FWD_LPHS_BF16_D64>(CDSSM_FWD_ARGS);
     if (D == 64)
@@ -1906,6 +1911,17 @@ int fused_fwd_entry(int dtype, const void* q, const void* k, const void* v, cons
 #undef CDSSM_FWD_ARGS
 }
 }  // namespace
+
+// The choice of cdssm_fused_scan_fwd for a shape (1 or 0), -1 for one that it refuses.
+extern "C" int cdssm_fused_scan_fwd_matrix_cores(int dtype, int64_t B, int64_t L, int64_t H, int64_t D, int64_t N,
+                                                 int64_t chunk) {
+  if ((dtype != 0 && dtype != 1) || B <= 0 || L <= 0 || H <= 0 || N != 2 || (D != 64 && D != 128) || chunk < 1 ||
+      chunk > 128 || B * H > 0x7fffffffLL || L > 0x7fffffffLL) {
+    cdssm_host::set_error("cdssm_fused_scan_fwd_matrix_cores: not a shape of the fused scan");
+    return CDSSM_EINVAL;
+  }
+  return takes_matrix_cores(dtype, B, L, H, D, chunk) ? 1 : 0;
+}
 
 extern "C" int cdssm_fused_scan_fwd(int dtype, const void* q, const void* k, const void* v,
                                     const void* beta, const void* sel_c, const void* dt,

@@ -360,6 +360,15 @@ int cdssm_fused_scan_fwd_stamped(int dtype, const void* q, const void* k, const 
 int cdssm_fused_scan_fwd_set_path(int mode);
 
 /*
+ * Which one-launch kernel cdssm_fused_scan_fwd runs for the shape under the
+ * present path setting on the current device (no counterpart in the reference;
+ * for tests and benchmarks): 1 the matrix-core one, 0 another form, -1 for a
+ * shape that it refuses.
+ */
+int cdssm_fused_scan_fwd_matrix_cores(int dtype, int64_t B, int64_t L, int64_t H, int64_t D, int64_t N,
+                                      int64_t chunk);
+
+/*
  * Look-back health (no counterpart in the reference, whose inter-chunk pass is
  * a separate serial launch, inter_chunk_scan.cu:201-234).  The one-launch
  * forward and the backward's one-launch correction adjoint + carry pass chunk

@@ -73,6 +73,14 @@ def oracle_fwd(x: dict, chunk_size=None):
                         d["omega"], d["c"], h0=d.get("h0"), chunk_size=chunk_size)
 
 
+def on_matrix_cores(cfg) -> bool:
+    """Whether the bf16 inference forward of this shape runs the matrix-core kernel under the present path setting."""
+    from cdssm_hip import _lib
+    st = _lib.load().cdssm_fused_scan_fwd_matrix_cores(1, cfg.B, cfg.L, cfg.H, cfg.D, cfg.N, cfg.D)
+    assert st >= 0, _lib.last_error()
+    return st == 1
+
+
 GRAD_NAMES = ("q", "k", "v", "beta", "sel_C", "dt", "r", "alpha", "omega")
 
 
