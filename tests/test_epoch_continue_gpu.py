@@ -1,14 +1,14 @@
 """Calls that reuse the look-back epoch left in their workspace (*_continue).
 
 The one-launch passes tag their look-back flags with a per-call epoch.  The
-plain entry points draw it with a one-thread kernel before the pass; the
-*_continue entry points, which PreparedForward / PreparedBackward use after
-their first call, run on the epoch that the previous call's last workgroup
-left in the workspace.  If that hand-over failed, a later call would read the
+plain entry points draw it on the host, or with a one-thread kernel before the
+pass where they are captured; the *_continue entry points, which
+PreparedForward / PreparedBackward use after their first call, run on the epoch
+that the previous call's last workgroup left in the workspace.  If that hand-over failed, a later call would read the
 previous call's flags as ready and fold stale chunk maps: its outputs would
 differ from a fresh call's.  These tests run many consecutive prepared calls
 with inputs rewritten in place and require each to be bit-identical to a
-plain call (own workspace, epoch kernel) on the same inputs; the kernels and
+plain call (own workspace, own epoch) on the same inputs; the kernels and
 their fixed fold order are the same, so any difference is a stale fold.
 Shapes: a one-round one-pass forward, a persistent (multi-round) one-pass
 forward, and the training forward with the backward's one-launch carry.
@@ -19,7 +19,7 @@ import contextlib
 import pytest
 import torch
 
-from _gpu_util import DEV, ScanConfig, cotangents, draw_inputs, log, to_dev
+from _gpu_util import DEV, ScanConfig, cotangents, draw_inputs, log, on_matrix_cores, to_dev
 
 pytestmark = pytest.mark.gpu
 
@@ -50,8 +50,10 @@ def _fresh_forward(static: dict):
     return y.cpu(), hf.cpu()
 
 
-@pytest.mark.parametrize("name,B,H,L", [("one round", 2, 16, 4096), ("persistent", 1, 32, 65536)])
-def test_continuing_forward_calls_equal_fresh_calls(name, B, H, L):
+@pytest.mark.parametrize("name,B,H,L,path", [("one round", 2, 16, 4096, "one_pass"),
+                                             ("persistent", 1, 32, 65536, "one_pass"),
+                                             ("matrix cores", 2, 16, 4096, "auto")])
+def test_continuing_forward_calls_equal_fresh_calls(name, B, H, L, path):
     """PreparedForward: the first call draws the epoch, the next seven reuse the
     previous call's; inputs cycle through four seeds (each seen twice)."""
     from cdssm_hip import lookback_status
@@ -59,7 +61,8 @@ def test_continuing_forward_calls_equal_fresh_calls(name, B, H, L):
     cfg = ScanConfig("c", B=B, H=H, L=L, D=64, h0_std=0.1)
     log(f"[continue fwd] {name}: B{B} H{H} L{L} D64 bf16 h0, eight prepared calls")
     static = to_dev(draw_inputs(cfg, seed=0))
-    with forward_path("one_pass"):
+    with forward_path(path):
+        assert on_matrix_cores(cfg) == (path == "auto")
         pf = PreparedForward(*[static[n] for n in TOKEN_INPUTS], static["c"], h0=static["h0"])
         for i, seed in enumerate((11, 12, 13, 14, 11, 12, 13, 14)):
             _rewrite(static, draw_inputs(cfg, seed=seed))
@@ -110,16 +113,18 @@ def test_continuing_training_forward_and_backward_equal_fresh_calls():
     assert lookback_status() == 0, "a look-back wait timed out"
 
 
-def test_first_call_under_capture_keeps_the_epoch_kernel():
+@pytest.mark.parametrize("path", ["one_pass", "auto"])
+def test_first_call_under_capture_keeps_the_epoch_kernel(path):
     """A PreparedForward whose first call is captured holds no executed call, so the
     graph keeps the plain entry (epoch kernel in the graph); replays on rewritten
     inputs and the eager calls after them equal fresh calls."""
     from cdssm_hip import lookback_status
     from cdssm_hip.scan import PreparedForward
     cfg = ScanConfig("g", B=2, H=16, L=4096, D=64)
-    log("[continue capture] B2 H16 L4096 D64 bf16, first call captured")
+    log(f"[continue capture] B2 H16 L4096 D64 bf16, first call captured ({path})")
     static = to_dev(draw_inputs(cfg, seed=0))
-    with forward_path("one_pass"):
+    with forward_path(path):
+        assert on_matrix_cores(cfg) == (path == "auto")
         _fresh_forward(static)  # fills the launcher's occupancy cache outside capture
         pf = PreparedForward(*[static[n] for n in TOKEN_INPUTS], static["c"])
         graph = torch.cuda.CUDAGraph()

@@ -17,8 +17,8 @@ import contextlib
 import pytest
 import torch
 
-from _gpu_util import (DEV, GRAD_NAMES, ScanConfig, cotangents, draw_inputs, log, oracle_fwd, oracle_grads, rel,
-                       select, state_norm_rel, to_dev)
+from _gpu_util import (DEV, GRAD_NAMES, ScanConfig, cotangents, draw_inputs, log, on_matrix_cores, oracle_fwd,
+                       oracle_grads, rel, select, state_norm_rel, to_dev)
 
 pytestmark = pytest.mark.gpu
 
@@ -43,15 +43,18 @@ def _rewrite(static: dict, x: dict) -> None:
         static["h0"].copy_(x["h0"].to(DEV))
 
 
-def test_captured_one_pass_forward_replays_match_oracle_c1():
-    """C1 (B8 H16 L4096 D64 bf16), one-pass forward captured once; three replays on
-    three input sets written in place; selected sequences checked against the oracle."""
+@pytest.mark.parametrize("path", ["one_pass", "auto"])
+def test_captured_one_pass_forward_replays_match_oracle_c1(path):
+    """C1 (B8 H16 L4096 D64 bf16), the one-launch forward captured once (the sequential one, and the default, which is
+    on the matrix cores); three replays on three input sets written in place; selected sequences checked against
+    the oracle."""
     from cdssm_hip import lookback_status
     from cdssm_hip.scan import PreparedForward
     cfg = ScanConfig("C1", B=8, H=16, L=4096, D=64)
-    log("[graph fwd] C1 B8 H16 L4096 D64 bf16, one-pass forward captured")
+    log(f"[graph fwd] C1 B8 H16 L4096 D64 bf16, one-launch forward captured ({path})")
     static = to_dev(draw_inputs(cfg, seed=0))
-    with forward_path("one_pass"):
+    with forward_path(path):
+        assert on_matrix_cores(cfg) == (path == "auto")
         pf = PreparedForward(*[static[n] for n in TOKEN_INPUTS], static["c"])
         pf()  # eager call first: fills the launcher's occupancy cache outside capture
         torch.cuda.synchronize()
@@ -78,7 +81,7 @@ def test_captured_one_pass_forward_replays_match_oracle_c1():
         log(f"   replay seed {seed}: rel err y {ey:.2e}  state-norm {en:.2e}")
         assert ey <= 2e-2 and en <= 1e-3, (seed, ey, en)
         # the same inputs through an eager call: identical bits (fixed fold order)
-        with forward_path("one_pass"):
+        with forward_path(path):
             pf()
         torch.cuda.synchronize()
         assert torch.equal(pf.y.cpu(), y) and torch.equal(pf.h_final.cpu(), hf), f"eager != replay (seed {seed})"

@@ -10,7 +10,7 @@ log / exp (2e-5) being the largest error, so 5e-5 of the largest state value.
 import pytest
 import torch
 
-from _gpu_util import DEV, ScanConfig, draw_inputs, log, oracle_fwd, rel, to_dev
+from _gpu_util import DEV, ScanConfig, draw_inputs, log, on_matrix_cores, oracle_fwd, rel, select, to_dev
 
 pytestmark = pytest.mark.gpu
 
@@ -20,6 +20,8 @@ KEYS = ("q", "k", "v", "beta", "sel_C", "dt", "r", "alpha", "omega")
 
 def run(x, chunk=None):
     from cdssm_hip import check_lookback, chunkwise_delta_scan
+    B, L, H, D = x["q"].shape
+    assert on_matrix_cores(ScanConfig("t", B=B, H=H, L=L, D=D))
     y, h = chunkwise_delta_scan(*[x[n] for n in KEYS], x["c"], h0=x.get("h0"), chunk_size=chunk)
     torch.cuda.synchronize()
     check_lookback()
@@ -36,6 +38,21 @@ def test_matches_oracle_at_the_edges_of_blocks_chunks_and_head_groups(B, H, L, D
     y, h = run(to_dev(x), chunk)
     yr, hr = oracle_fwd(x, chunk)
     assert rel(y, yr) <= TOL_Y and rel(h, hr) <= TOL_H, (rel(y, yr), rel(h, hr))
+
+
+@pytest.mark.parametrize("D,segments", [(64, 15), (64, 17), (64, 70), (128, 66)])
+def test_matches_oracle_over_group_and_anchor_ends(D, segments):
+    """More segments than are folded one by one (15), than one group, and than lie between two anchors (64): heads
+    with a slow decay, so that a state entering the first segments reaches the last ones.  Its factor is a product of
+    L transitions, each formed in fp32 with a hardware reciprocal and exponential: off by 2^-23 each, L 2^-23 in
+    all; a map folded twice or not at all is wrong by the values' size."""
+    log(f"[mfma forward] {segments} segments D{D}")
+    x = draw_inputs(ScanConfig("t", B=2, H=4, L=segments * 4 * D - 5, D=D, h0_std=1.0), seed=segments)
+    x["alpha"], x["omega"], x["r"] = x["alpha"] * 1e-4, x["omega"] * 1e-3, x["r"] * 1e-3
+    y, h = run(to_dev(x))
+    yr, hr = oracle_fwd(select(x, [1], [2]))
+    ey, eh, tol = rel(y[1:2, :, 2:3], yr), rel(h[1:2, 2:3], hr), x["q"].shape[1] * 2.0 ** -23
+    assert ey <= TOL_Y + tol and eh <= TOL_H + tol, (ey, eh, tol)
 
 
 @pytest.mark.parametrize("alpha,omega", [(3.0, 0.02), (1.0, 0.0), (10.0, 0.1)])
