@@ -22,11 +22,14 @@
 // A call is one latency chain: its weight rows, its activation rows, the sum.
 // What bounds it is how many loads one CU has to issue and return, so the rows
 // are split over the CUs as far as one round of workgroups takes them
-// (kOneRound).  Measured on MI355X at M = 64, K = 1024, us per call back to
+// (one per CU).  Measured on MI355X at M = 64, K = 1024, us per call back to
 // back, for 16 / 32 / 64 rows per workgroup: N = 1024 4.5 / 5.2 / 7.0,
 // N = 1552 6.2 / 5.3 / 6.9, N = 2048 6.2 / 5.5 / 7.3, N = 3104 9.7 / 8.6 / 7.9;
 // with the norm at N = 1024 5.2 / 6.0 / 8.0, N = 3104 10.9 / 8.9 / 8.9.  At
-// M = 16, K = 2048, N = 4096 7.5 / 7.7 / 9.0.  (Always 64 rows before.)
+// M = 16, K = 2048, N = 4096 7.5 / 7.7 / 9.0.  (Always 64 rows before.)  Where the
+// line lies, 256 CUs, M = 64, K = 1024, in a graph over 8 weights, 16 / 32 / 64
+// rows: N = 1024 (256 workgroups of 16 rows) 4.1 / - / 6.8, N = 1040 (260) 5.7 / 5.0
+// / 6.8, N = 1136 (284) 5.8 / 5.0 / 6.8, N = 1440 (360) 6.0 / 5.3 / 7.1.
 //
 // Fragment layouts of v_mfma_f32_16x16x32_bf16 (checked on MI355X):
 //   A (16 x 32): lane l holds row l % 16, k = 8 (l / 16) .. + 8
@@ -45,9 +48,6 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kCols = 16;   // output columns per workgroup
 constexpr int kMaxRows = 64;
-// Workgroups that count as one round: one per CU (256), and an eighth of the CUs may hold a second one
-// (N = 1136, M = 64: 284 workgroups of 16 rows 6.0 us, 142 of 32 rows 6.25; N = 1552: 388 of 16 6.2, 194 of 32 5.3).
-constexpr int64_t kOneRound = 288;
 constexpr int kUnroll = 4;  // k-steps (of 32) whose loads are issued together
 
 __device__ __forceinline__ uint4 ld16(const uint16_t* p) { return *reinterpret_cast<const uint4*>(p); }
@@ -290,7 +290,7 @@ static int skinny_gemm(const char* op, int dtype, const void* X, int64_t ldx, co
   using W4 = std::integral_constant<int, 4>;
   auto rows = [&](auto norm, auto waves) {
     const int64_t nt = (N + sg::kCols - 1) / sg::kCols, mt = (M + 15) / 16;
-    const int64_t cap = sg::kOneRound;
+    const int64_t cap = cdssm_host::device_cus();  // one round: a workgroup per CU
     if (nt * mt <= cap) return go(norm, waves, std::integral_constant<int, 1>{});
     if (nt * ((mt + 1) / 2) <= cap) return go(norm, waves, std::integral_constant<int, 2>{});
     go(norm, waves, std::integral_constant<int, sg::kMaxRows / 16>{});

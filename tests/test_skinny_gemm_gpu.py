@@ -139,3 +139,27 @@ def test_conv_step_in_the_product(M, N, col, C, taps):
         want = skinny_linear(x, w, b, norm_weight=nw, eps=1e-5)
         assert torch.equal(y, want)
         assert torch.equal(yc, conv1d_silu_step(want[:, col:col + C], win2, cw, cb)) and torch.equal(win, win2)
+
+
+@pytest.mark.parametrize("K", [128, 384, 512])
+@pytest.mark.parametrize("norm", [True, False])
+@pytest.mark.parametrize("M,N,col,C,taps", [(64, 3104, 1024, 1024, 4), (40, 1040, 16, 1000, 4), (9, 70, 5, 60, 3)])
+def test_conv_step_with_four_waves_and_without_a_norm(M, N, col, C, taps, norm, K):
+    """K not a multiple of 256 (four waves to a workgroup), at 64, 32 and 16 rows per workgroup, with and without the
+    norm weight, through the C entry: equal bits to the product and the step in their own launches."""
+    from cdssm_hip import _lib
+    from cdssm_hip.lm import conv1d_silu_step, skinny_linear
+    g = torch.Generator().manual_seed(K + N)
+
+    def rnd(*s):
+        return torch.randn(*s, generator=g).to(torch.bfloat16).to(DEV)
+
+    x, w, b, nw = rnd(M, K), rnd(N, K), rnd(N), rnd(K) if norm else None
+    cw, cb, win = rnd(C, taps), rnd(C), rnd(M, taps - 1, C)
+    y, yc, win2 = rnd(M, N), rnd(M, C), win.clone()
+    _lib.check(_lib.load().cdssm_skinny_gemm_conv_step(
+        1, _lib.ptr(x), K, _lib.ptr(w), K, _lib.ptr(b), _lib.ptr(nw), 1e-5, _lib.ptr(y), N, M, N, K, col,
+        _lib.ptr(win), _lib.ptr(cw), _lib.ptr(cb), _lib.ptr(yc), C, taps, _lib.stream_of(DEV)), "conv step")
+    want = skinny_linear(x, w, b, norm_weight=nw, eps=1e-5)
+    assert torch.equal(y, want)
+    assert torch.equal(yc, conv1d_silu_step(want[:, col:col + C], win2, cw, cb)) and torch.equal(win, win2)
