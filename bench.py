@@ -623,11 +623,11 @@ def time_lm_decode(steps=20, warmup=3, B=64, prompt=2048):
     return {"workload": f"config 4: LM decode step B{B} from a {prompt}-token prefill, 24 layers, bf16",
             "ms_per_step": ms, "tokens_per_s": B / (ms * 1e-3), "eager_ms_per_step": ms_eager,
             "prefill_ms": p0.elapsed_time(p1), "weight_bytes": wbytes, "weight_read_GBs": wbytes / (ms * 1e-3) / 1e9,
-            "note": "one HIP graph per step (DecodeGraph); per layer 5 launches: RMSNorm + in_proj (skinny GEMM), "
-                    "conv step, stacked gate/Q projection (skinny GEMM), one tail kernel (dynamics, K/Q norm, value "
-                    "residual, scan step, shortcut, then readout_proj and the GroupNorm step of the batch row: "
-                    "cdssm_decode_block_tail), out_proj with the residual (skinny GEMM); then the final RMSNorm and "
-                    "the tied head (library GEMM)"}
+            "note": "one HIP graph per step (DecodeGraph); per layer 4 launches: RMSNorm + in_proj + conv step "
+                    "(cdssm_skinny_gemm_conv_step), stacked gate/Q projection (skinny GEMM), one tail kernel (dynamics, "
+                    "K/Q norm, value residual, scan step, shortcut, then readout_proj and the GroupNorm step of the "
+                    "batch row: cdssm_decode_block_tail), out_proj with the residual (skinny GEMM); then the final "
+                    "RMSNorm and the tied head (library GEMM)"}
 
 
 def time_lm_forward(steps=5, warmup=2, state_dim=2):

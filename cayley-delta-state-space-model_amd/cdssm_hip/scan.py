@@ -265,8 +265,8 @@ FORWARD_PATHS = {"auto": 0, "four_launch": 1, "one_pass": 2, "four_launch_mfma":
 
 # Bumped by every set_forward_path call.  A prepared call continues on the
 # look-back epoch its previous call left only while the path setting is the one
-# that call ran under: a call made under another setting may have taken the
-# multi-launch passes, which never write the workspace's control block.
+# that call ran under: a call made under another setting may have run another
+# kernel on the workspace, and left it the epoch of that one or none.
 _path_generation = [0]
 
 
@@ -275,13 +275,16 @@ def set_forward_path(path: str) -> str:
 
     "auto" (default) takes a one-launch forward where one round of resident
     workgroups holds every segment of 4 chunks (for scan-level bf16 inference
-    the matrix-core form, whose y differs from the sequential forms' by the
-    order of its sums; else the sequential one-pass, for inference also where
-    it fills whole persistent rounds), else the four-launch scan; "four_launch" always takes the multi-launch passes; "one_pass" requires
-    the sequential one-launch passes (calls they cannot serve raise); "four_launch_mfma"
-    takes the multi-launch passes with the correction as the chunked MFMA
-    pass (bf16 inference forward, chunk a multiple of 16 up to 128; other calls
-    raise).  Process-wide; the same choice applies to the backward's correction
+    the matrix-core form; else the sequential one-pass, for inference also where
+    it fills whole persistent rounds), else the four-launch scan; "four_launch"
+    always takes the multi-launch passes; "one_pass" requires the sequential
+    one-launch passes (calls they cannot serve raise); "four_launch_mfma" takes
+    the multi-launch passes with the correction as the chunked MFMA pass (bf16
+    inference forward, chunk a multiple of 16 up to 128; other calls raise).
+    The matrix-core form sums in fp32 as the sequential ones do, in another
+    order.  So the bits of an inference call depend on whether its B, L and H
+    fit one round, and need not be the training forward's, which is sequential.
+    Process-wide; the same choice applies to the backward's correction
     adjoint + reverse carry.
     """
     if path not in FORWARD_PATHS:

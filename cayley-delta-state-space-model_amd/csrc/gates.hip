@@ -78,8 +78,8 @@ struct WideRow {
 
 // NH = N / 2 pairs: for the usual state sizes a constant, with the token's gates requested before any is used
 // and its A_bar and vp rows stored whole; 0 for every other N, a pair's loads after the previous pair's
-// arithmetic and 2-byte stores.  B 4, L 2048, H 24, N 16, bf16 on MI355X: 18.9 -> 14.2 us; B 8, L 2048, H 16,
-// N 2: 8.0 -> 7.2 us.
+// arithmetic and 2-byte stores.  bf16 on MI355X, calls back to back: B 4, L 2048, H 24, N 16 18.3 -> 12.7 us; B 8,
+// L 2048, H 16, N 16 21.6 -> 16.0, N 2 6.8 -> 6.4.
 template <typename T, int NH>
 __global__ __launch_bounds__(256) void dynamics_fwd_kernel(
     const typename T::raw* __restrict__ gate, const float* __restrict__ log_dt_scale,
@@ -128,7 +128,7 @@ __global__ __launch_bounds__(256) void dynamics_fwd_kernel(
 }
 
 // NH as in the forward: the gates, and the token's gradient rows whole, are requested before any is used.
-// B 8, L 2048, H 16, N 16, bf16 on MI355X: 29.4 -> 24.7 us.
+// bf16 on MI355X, calls back to back: B 8, L 2048, H 16, N 16 34.1 -> 31.6 us; B 4, H 24 28.0 -> 25.6.
 template <typename T, int NH>
 __global__ __launch_bounds__(256) void dynamics_bwd_kernel(
     const typename T::raw* __restrict__ gA, const typename T::raw* __restrict__ gvp,
